@@ -18,7 +18,10 @@
 //      - attn_mfma_kernel: one workgroup per (row, partition, kv head), its
 //        waves merged in LDS, partitions merged by attn_reduce_kernel;
 //  * attn_valu_kernel - any group and f32 KV: lanes split a token row into
-//    4-element slices, dot products reduce across the row's lanes.
+//    4-element slices, dot products reduce across the row's lanes.  The
+//    row-block kernels (rows.hip) serve most of its shapes faster; it keeps the
+//    shortest f32 calls, head sizes that are not whole 8-element pieces (f16,
+//    e4m3) and buffers that are not 16-byte aligned.
 // All keep the online-softmax state of Reference/paged_attention_sim.py:94-123
 // (in log2 units).
 #include "attention_body.h"
@@ -213,9 +216,21 @@ static hipError_t launch_valu(const AttnParams &p, hipStream_t stream, const Ker
     return hipGetLastError();
 }
 
+hipError_t launch_reduce(const AttnParams &p, int32_t dtype, hipStream_t stream, const KernelTable *kt) {
+    const dim3 grid((p.num_heads + 3) / 4, p.rows);
+    hipError_t e;
+    if (via_module(kt, kt ? kt->reduce[dtype != kF32] : nullptr, &e, grid, dim3(256), stream, p)) return e;
+    if (dtype == kF32)
+        hipLaunchKernelGGL((attn_reduce_kernel<float>), grid, dim3(256), 0, stream, p);
+    else
+        hipLaunchKernelGGL((attn_reduce_kernel<f16>), grid, dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
 hipError_t launch_attention(const AttnParams &p_in, int32_t dtype, bool use_mfma, hipStream_t stream,
                             hipEvent_t after_main, const KernelTable *kt) {
     if (p_in.rows <= 0) return hipSuccess;
+    if (!use_mfma && p_in.row_blocks) return launch_rows(p_in, dtype, stream, after_main, kt);
     AttnParams p = p_in;
     p.epoch = next_launch_epoch();
     // masked lanes of the MFMA kernel read a lane-group slice of one token row
@@ -236,13 +251,7 @@ hipError_t launch_attention(const AttnParams &p_in, int32_t dtype, bool use_mfma
     if (after_main) (void)hipEventRecord(after_main, stream);
     // stream-K (MFMA) and the VALU kernel with counters merge in the kernel
     if (p.max_parts <= 1 || p.seg_count != nullptr || p.valu_wg) return e;
-    dim3 grid((p.num_heads + 3) / 4, p.rows);
-    if (via_module(kt, kt ? kt->reduce[dtype != kF32] : nullptr, &e, grid, dim3(256), stream, p)) return e;
-    if (dtype == kF32)
-        hipLaunchKernelGGL((attn_reduce_kernel<float>), grid, dim3(256), 0, stream, p);
-    else
-        hipLaunchKernelGGL((attn_reduce_kernel<f16>), grid, dim3(256), 0, stream, p);
-    return hipGetLastError();
+    return launch_reduce(p, dtype, stream, kt);
 }
 
 }  // namespace pam

@@ -87,6 +87,8 @@ struct AttnParams {
     // VALU kernel: 1 runs a (row, head group)'s partitions as the waves of one
     // workgroup (attn_valu_wg_kernel), merged in LDS
     int32_t valu_wg;
+    // 1: the row-block kernels (rows.hip) in place of the VALU kernel
+    int32_t row_blocks;
 };
 
 // Entry points of a loaded code object (libpam_kernels.hsaco, module_entry.hip).
@@ -101,6 +103,8 @@ struct KernelTable {
     hipFunction_t mixed[2];       // one-launch mixed step: f16, e4m3
     hipFunction_t valu[3][4];     // VALU rows: [f32, f16, e4m3 KV][1, 2, 4, 8 heads per wave]
     hipFunction_t valu_wg[3][2];  // their workgroup form: [KV][1, 2 heads per wave]
+    // row blocks (rows.hip): [f32, f16, e4m3 KV][head size up to 32, 64, 96, 128, 256]
+    hipFunction_t prefill_rows[3][5], decode_rows[3][5];
     hipFunction_t reduce[2];      // split-context reduce: f32, f16 outputs
     hipFunction_t append[3];      // append copy in 16-, 4- or 2-byte pieces
     hipFunction_t append_batch[3];
@@ -264,6 +268,17 @@ hipError_t launch_mfma_loop(int blocks, int iters, float *sink, hipStream_t stre
 hipError_t launch_synth_normal(void *dst, int32_t dtype, uint64_t n, uint64_t seed, uint64_t stream, float stddev,
                                int64_t outlier_stream, float outlier_frac, hipStream_t s);
 
+// Split-context reduce of rows whose partials are in p.part_o / p.part_ml.
+hipError_t launch_reduce(const AttnParams &p, int32_t dtype, hipStream_t stream, const KernelTable *kt);
+// Attention over blocks of query rows with f32 probabilities on the matrix units
+// (rows.hip): a prefill (kRowPrefill: 32 rows of one sequence per block) or decode
+// and ragged rows (up to 16 heads per kv-head slot), any group and block size.
+// The caller sets p.row_blocks, p.part_tokens (a multiple of 16), p.max_parts and, when max_parts > 1, the partials, which the reduce
+// launched after it merges.
+bool rows_supported(const AttnParams &p, int32_t dtype);
+int32_t prefill_rows_part_tokens(const AttnParams &p, int32_t dtype, int32_t cus);
+hipError_t launch_rows(const AttnParams &p, int32_t dtype, hipStream_t stream, hipEvent_t after_main,
+                       const KernelTable *kt = nullptr);
 // Dense chunked-prefill (MFMA, f16): rows [q_offset, q_offset + T) of one sequence.
 // Dense prefill (MFMA): f16 or e4m3 KV, d = 128; Q and O f16.
 hipError_t launch_prefill_mfma(const AttnParams &p, int32_t dtype, hipStream_t stream,

@@ -12,6 +12,7 @@
 #include "../kernels/attention_body.h"
 #include "../kernels/mixed_body.h"
 #include "../kernels/prefill_body.h"
+#include "../kernels/rows_body.h"
 #include "../kernels/stage_body.h"
 #include "../kernels/valu_body.h"
 
@@ -46,6 +47,14 @@ namespace pam {
         __shared__ float wg_lds[kValuWgLds<NH>];                                                             \
         valu_body<KV, QT, NH, true>(p, lanes_per_row, wg_lds);                                              \
     }
+#define PAM_ROWS_ENTRY(NAME, BODY, RB, KV, QT, NT)                                                      \
+    extern "C" __global__ __launch_bounds__(64 * kRowsWaves, (NT <= 4 ? 2 : 1)) void NAME(AttnParams p) { \
+        __shared__ __attribute__((aligned(16))) float lds[kRowsLds<NT, (RB)>];                            \
+        BODY<KV, QT, NT>(p, lds);                                                                       \
+    }
+#define PAM_ROWS_ENTRIES(KVNAME, KV, QT, NT, DIM)                                                       \
+    PAM_ROWS_ENTRY(pam_prefill_rows_##KVNAME##_d##DIM, prefill_rows_body, (kPrefillRowsRB<KV, NT>), KV, QT, NT) \
+    PAM_ROWS_ENTRY(pam_decode_rows_##KVNAME##_d##DIM, decode_rows_body, 1, KV, QT, NT)
 #define PAM_APPEND_ENTRY(NAME, CH)                                                                          \
     extern "C" __global__ __launch_bounds__(256) void NAME(AppendParams p, int64_t chunks_per_row,        \
                                                            int64_t total) {                               \
@@ -97,6 +106,22 @@ PAM_PREFILL_ENTRY(pam_prefill_e4m3_d128, 128, false, uint8_t)
 PAM_PREFILL_ENTRY(pam_prefill_f16_d64, 64, false, f16)
 PAM_PREFILL_ENTRY(pam_prefill_fused_f16_d64, 64, true, f16)
 PAM_PREFILL_ENTRY(pam_prefill_e4m3_d64, 64, false, uint8_t)
+// blocks of query rows with f32 probabilities (rows_body.h), by KV type and head size
+PAM_ROWS_ENTRIES(f32, float, float, 1, 32)
+PAM_ROWS_ENTRIES(f32, float, float, 2, 64)
+PAM_ROWS_ENTRIES(f32, float, float, 3, 96)
+PAM_ROWS_ENTRIES(f32, float, float, 4, 128)
+PAM_ROWS_ENTRIES(f32, float, float, 8, 256)
+PAM_ROWS_ENTRIES(f16, f16, f16, 1, 32)
+PAM_ROWS_ENTRIES(f16, f16, f16, 2, 64)
+PAM_ROWS_ENTRIES(f16, f16, f16, 3, 96)
+PAM_ROWS_ENTRIES(f16, f16, f16, 4, 128)
+PAM_ROWS_ENTRIES(f16, f16, f16, 8, 256)
+PAM_ROWS_ENTRIES(e4m3, uint8_t, f16, 1, 32)
+PAM_ROWS_ENTRIES(e4m3, uint8_t, f16, 2, 64)
+PAM_ROWS_ENTRIES(e4m3, uint8_t, f16, 3, 96)
+PAM_ROWS_ENTRIES(e4m3, uint8_t, f16, 4, 128)
+PAM_ROWS_ENTRIES(e4m3, uint8_t, f16, 8, 256)
 // one-launch mixed step
 PAM_MIXED_ENTRY(pam_mixed_step_f16_d128, f16)
 PAM_MIXED_ENTRY(pam_mixed_step_e4m3_d128, uint8_t)

@@ -323,6 +323,18 @@ int32_t Context::choose_part_tokens(int64_t items_per_part, int64_t max_tiles, b
     return (int32_t)(tpp * 16);
 }
 
+// Decode rows that the VALU kernel's workgroup form still serves faster than the
+// row-block kernel: f32, one query head per kv head, at most 256 tokens.  There
+// the matrix form computes 16 rows for one, and a tile's f32 matrix time is the
+// longest step of the call.  Measured on gfx950 (µs per call, VALU / row blocks):
+// 8/8 d = 128: B = 4 L <= 200 9.5 / 10.1, B = 64 L <= 100 10.6 / 12.2, B = 128
+// L <= 200 26.0 / 30.8; d = 256 B = 4 L <= 200 14.1 / 17.0; 16/16 d = 64: B = 4
+// L <= 200 8.6 / 7.6, B = 64 15.7 / 16.7; 8/4 d = 128 B = 32 L <= 200 12.8 / 10.2.
+static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles) {
+    return dtype == kF32 && p.num_heads == p.num_kv_heads && max_tiles <= kValuWgMaxParts &&
+           (p.head_dim > 64 || (int64_t)p.rows * p.num_heads >= 512);
+}
+
 // Split-context set-up of a row launch (p.rows and the shape already filled).
 // The MFMA kernel runs in its stream-K form when the rows fit it: partial slots
 // in the workspace plus the counters, no reduce kernel.  Otherwise rows are cut
@@ -332,6 +344,7 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
                             char *fixed) {
     p.seg_count = nullptr;
     p.valu_wg = 0;
+    p.row_blocks = 0;
     int64_t slots = 0, counters = 0;
     // `fixed`: the allocation-free scratch (kNoAllocScratchBytes, laid out as
     // zero page | counters | partials); requests that do not fit it are refused
@@ -372,6 +385,42 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
         }
         p.part_ml = p.part_o + slots * p.head_dim;
         p.part_bytes = (uint32_t)bytes;
+        return bytes;
+    }
+    if (!use_mfma && p.mode != kRowPrefill && decode_kernel_choice != 1 && rows_supported(p, dtype) &&
+        !valu_rows_win(p, dtype, max_tiles)) {
+        // Row-block kernel: one workgroup per (row, slot of up to 16 heads,
+        // partition).  A row is cut until there are about 8 workgroups per CU, to
+        // no less than 256 tokens (a partition's start and the reduce cost more
+        // than they spread), or 128 for few pairs with long contexts.  Measured on
+        // gfx950 (µs per call, least partition 16 / 8 / 4 tiles of 16 tokens):
+        // f32 8/8 d = 128 B = 4 L <= 200 10.1 / 11.7 / 10.9, f16 16/16 d = 256
+        // B = 16 L <= 1000 50.1 / 59.0 / 58.9, f16 8/8 d = 128 B = 1 L <= 4000
+        // 13.7 / 12.7 / 12.7, f32 32/8 B = 1 L <= 5598 14.5 / 12.4 / 13.7;
+        // 2 / 4 / 8 workgroups per CU: e4m3 12/4 d = 128 B = 205 L <= 4000
+        // 227 / 189 / 172, f32 8/8 B = 64 L <= 2000 132 / 131 / 117.
+        const int64_t pairs = (int64_t)p.rows * p.num_kv_heads * ceil_div(p.num_heads / p.num_kv_heads, 16);
+        const int64_t least = pairs <= 64 && max_tiles >= 48 ? 8 : 16;
+        int64_t tpp = max_tiles;
+        while (tpp > least && pairs * ceil_div(max_tiles, tpp) < 8 * (int64_t)cus_) tpp = (tpp + 1) / 2;
+        if (part_tokens_override > 0) tpp = std::max<int32_t>(1, part_tokens_override / 16);
+        auto bytes_of = [&](int64_t t) {
+            return t >= max_tiles ? (int64_t)0
+                                  : p.rows * (int64_t)p.num_heads * ceil_div(max_tiles, t) * (p.head_dim + 2) * 4;
+        };
+        while (fixed && bytes_of(tpp) > fixed_parts) tpp *= 2;
+        p.row_blocks = 1;
+        p.part_tokens = (int32_t)(std::min(tpp, max_tiles) * 16);
+        p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(max_tiles, tpp));
+        const int64_t bytes = bytes_of(tpp);
+        if (bytes == 0) return 0;
+        if (fixed) {
+            p.part_o = reinterpret_cast<float *>(fixed + kNoAllocZeroBytes + kNoAllocCounterBytes);
+        } else {
+            reserve_workspace((size_t)bytes);
+            p.part_o = static_cast<float *>(workspace_.ptr);
+        }
+        p.part_ml = p.part_o + (int64_t)p.rows * p.num_heads * p.max_parts * p.head_dim;
         return bytes;
     }
     p.part_tokens = choose_part_tokens(waves, max_tiles, use_mfma);
@@ -536,6 +585,11 @@ void Context::module_load(const char *path) {
     for (int k = 0; k < 3; k++)
         for (int h = 0; h < 2; h++)
             t.valu_wg[k][h] = get(("pam_decode_valu_wg_" + std::string(kv_names[k]) + "_h" + std::to_string(heads[h])).c_str());
+    static const char *dims[5] = {"32", "64", "96", "128", "256"};
+    for (int k = 0; k < 3; k++)
+        for (int w = 0; w < 5; w++)
+            t.prefill_rows[k][w] = get(("pam_prefill_rows_" + std::string(kv_names[k]) + "_d" + dims[w]).c_str()),
+            t.decode_rows[k][w] = get(("pam_decode_rows_" + std::string(kv_names[k]) + "_d" + dims[w]).c_str());
     t.reduce[0] = get("pam_reduce_f32");
     t.reduce[1] = get("pam_reduce_f16");
     static const char *piece[3] = {"16", "4", "2"};
@@ -1031,6 +1085,20 @@ void Context::validate_prefill(const pam_prefill_request &r) {
         throw invalid_configuration("prefill request has a null buffer.");
 }
 
+// Short prefills that the VALU kernel's workgroup form (one or two heads per
+// wave, at most 256 keys) still serves faster than the row-block kernel, whose
+// tiles cost the same for one row as for 32.  Measured on gfx950 (µs per call,
+// VALU / row blocks): f32 8/8 d = 128: 64 tokens 7.7 / 12.1, 32 after 200
+// 10.9 / 15.7, 64 after 100 15.1 / 16.3, 128 22.9 / 16.1; f32 16/8 d = 128: 64
+// 10.3 / 12.1, 64 after 100 20.5 / 16.7; f16 8/8 d = 96: 16 after 100 9.3 / 11.8,
+// 64 9.1 / 8.8; e4m3 8/4 d = 96: 8 tokens 9.9 / 8.3.
+static bool valu_prefill_wins(const pam_layer_spec &l, int64_t rows, int64_t kv_len) {
+    const int32_t G = l.num_heads / l.num_kv_heads;
+    const int64_t pairs = rows * l.num_heads * kv_len;
+    if (kv_len > 16 * kValuWgMaxParts || l.data_type == kFP8) return false;
+    return l.data_type == kF32 ? (G == 1 || G == 2) && pairs < 70000 : G == 1 && pairs < 31000;
+}
+
 Context::PrefillPlan Context::plan_prefill(const pam_prefill_request &r) {
     const pam_layer_spec &l = r.layer;
     const int32_t G = l.num_heads / l.num_kv_heads;
@@ -1069,6 +1137,10 @@ Context::PrefillPlan Context::plan_prefill(const pam_prefill_request &r) {
         const DensePlan d = plan_dense_prefill(p, &ch, 1, sl);
         bind_dense_prefill(p, d, static_cast<const char *>(stage(4, sl.blob.data(), sl.blob.size())));
         pl.tmp = d.tmp;
+    } else if (!pl.use_mfma && decode_kernel_choice != 1 && rows_supported(p, l.data_type) &&
+               !valu_prefill_wins(l, r.seq_len, pl.kv_len)) {
+        pl.blocks = true;
+        pl.tmp = plan_prefill_rows(p, l.data_type);
     } else {
         const int64_t waves = (int64_t)r.seq_len * (pl.use_mfma ? l.num_kv_heads : l.num_heads / nh);
         pl.tmp = plan_split(p, l.data_type, pl.use_mfma, max_tiles, waves);
@@ -1076,10 +1148,32 @@ Context::PrefillPlan Context::plan_prefill(const pam_prefill_request &r) {
     return pl;
 }
 
+// Partitions of a row-block prefill and the workspace of their partials, which
+// attn_reduce_kernel merges.  Returns the workspace bytes (0: one partition).
+int64_t Context::plan_prefill_rows(AttnParams &p, int32_t dtype) {
+    p.seg_count = nullptr;
+    p.valu_wg = 0;
+    p.row_blocks = 1;
+    p.part_tokens = part_tokens_override > 0 ? std::max<int32_t>(16, part_tokens_override / 16 * 16)
+                                             : prefill_rows_part_tokens(p, dtype, cus_);
+    const int64_t kv_len = (int64_t)p.q_offset + p.rows;
+    const int64_t k_lo = p.window > 0 && kv_len > p.window ? kv_len - p.window : 0;
+    p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(ceil_div(kv_len, 16) - k_lo / 16, p.part_tokens / 16));
+    if (p.max_parts <= 1) return 0;
+    const int64_t slots = (int64_t)p.rows * p.num_heads * p.max_parts;
+    const int64_t bytes = slots * ((int64_t)p.head_dim + 2) * 4;
+    reserve_workspace((size_t)bytes);
+    p.part_o = static_cast<float *>(workspace_.ptr);
+    p.part_ml = p.part_o + slots * p.head_dim;
+    return bytes;
+}
+
 void Context::launch_prefill_plan(const PrefillPlan &pl, int32_t dtype, bool mark_mid) {
     hipEvent_t mid = gpu_timing && mark_mid ? evmid_ : nullptr;
     if (pl.dense)
         check_launch([&] { return launch_prefill_mfma(pl.p, dtype, stream(), ktab()); }, "prefill");
+    else if (pl.blocks)
+        check_launch([&] { return launch_rows(pl.p, dtype, stream(), mid, ktab()); }, "prefill");
     else
         check_launch([&] { return launch_attention(pl.p, dtype, pl.use_mfma, stream(), mid, ktab()); }, "prefill");
 }

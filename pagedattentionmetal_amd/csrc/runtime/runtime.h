@@ -219,8 +219,10 @@ class Context {
     struct PrefillPlan {
         AttnParams p;
         bool dense, use_mfma;
+        bool blocks;  // row-block prefill (launch_prefill_rows)
         int64_t tmp, kv_len;
     };
+    int64_t plan_prefill_rows(AttnParams &p, int32_t dtype);
     PrefillPlan plan_prefill(const pam_prefill_request &r);
     void launch_prefill_plan(const PrefillPlan &pl, int32_t dtype, bool mark_mid = true);
     AppendParams append_params(const pam_append_request &r);

@@ -1,0 +1,187 @@
+"""The row-block kernels (rows.hip): prefill of f32 caches and of the f16 / e4m3
+head and block sizes the dense kernel does not take; decode of f32 caches, small
+head groups and those sizes.  Parity with the oracle at the edges of their blocks
+(32 rows, 16 heads), tiles (16 keys), partitions and head-size tiles; keys that
+hold Inf or NaN reach exactly the rows that see them, as on the VALU kernel; the
+code object runs them bit for bit."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import TOL, make_case, row_rel_err, to_dev, to_host
+from test_gpu_kernels import build_fp8, layer
+
+pytestmark = pytest.mark.gpu
+
+IO = {0: np.float32, 1: np.float16, 2: np.float16}
+
+
+def _engine():
+    from pagedattentionmetal_amd import PagedAttentionEngine
+    e = PagedAttentionEngine()
+    e.set_graceful_degradation(False)
+    return e
+
+
+def _prefill(eng, q, kd, vd, bt, T, lay, causal, off, ks=None, vs=None):
+    import torch
+    out = torch.full(q.shape, 7.0, dtype=torch.float32 if q.dtype == np.float32 else torch.float16, device="cuda")
+    eng.prefill(to_dev(q), kd, vd, to_dev(bt), out, T, lay, causal=causal, q_offset=off, k_scale=ks, v_scale=vs)
+    return to_host(out)
+
+
+@pytest.mark.parametrize("dtype,T,off,H,hkv,d,bs,causal,window,part", [
+    (0, 32, 0, 8, 8, 128, 16, True, 0, 0),
+    (0, 33, 31, 8, 8, 128, 16, True, 0, 0),      # a second block of one row, a second tile of one key
+    (0, 31, 1000, 8, 2, 64, 16, True, 0, 0),     # several partitions and the reduce
+    (0, 70, 45, 6, 2, 80, 12, True, 0, 48),      # G = 3, head size between tiles, short partitions
+    (0, 5, 300, 4, 4, 256, 8, True, 0, 0),
+    (0, 90, 10, 4, 1, 32, 1, False, 0, 0),       # one-token blocks, not causal
+    (0, 200, 0, 4, 4, 36, 16, True, 77, 0),      # rows before the window see no key
+    (0, 1, 0, 2, 2, 4, 16, True, 0, 0),          # one row, one key, one slice
+    (1, 130, 77, 12, 4, 96, 16, True, 0, 0),
+    (1, 65, 0, 40, 2, 64, 16, True, 0, 0),       # more than 16 heads a kv head
+    (1, 47, 500, 8, 8, 128, 24, True, 100, 0),   # a block size that is not a power of two
+    (2, 64, 33, 8, 2, 96, 16, True, 0, 0),
+    (2, 40, 0, 4, 4, 160, 4, False, 0, 0),
+])
+def test_rows_parity(dtype, T, off, H, hkv, d, bs, causal, window, part):
+    rng = np.random.default_rng(900 + T + d)
+    eng = _engine()
+    _, k, v, bt, lens = make_case(rng, 1, H, hkv, d, bs, dtype, [off + T])
+    q = rng.standard_normal((T, H, d)).astype(IO[dtype])
+    if dtype == 2:
+        kd, vd, ksd, vsd, k, v, ks, vs = build_fp8(eng, rng, k, v, bt, lens, hkv, d, bs)
+        ks, vs = ks.view(np.uint16), vs.view(np.uint16)
+    else:
+        kd, vd, ksd, vsd, ks, vs = to_dev(k), to_dev(v), None, None, None, None
+    eng.set_partition_tokens(part)
+    o = _prefill(eng, q, kd, vd, bt[0], T, layer(H, hkv, d, bs, dtype, window), causal, off, ksd, vsd).astype(np.float64)
+    ref = oracle.prefill(dtype, q, k, v, bt[0], off, causal=causal, window=window, k_scale=ks, v_scale=vs, n_threads=8)
+    fin = np.isfinite(ref).all(axis=-1)
+    assert np.isnan(o[~fin]).all(), "rows with no key in range are 0/0"
+    assert row_rel_err(o[fin], ref[fin]) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,d", [(0, 128), (0, 40), (1, 96)])
+def test_rows_inf_and_nan_stay_with_the_rows_that_see_them(dtype, d):
+    """Against the VALU kernel (set_decode_kernel(1)) with single Inf and NaN elements
+    of K and V at keys that some rows of a block mask."""
+    T, off, H, hkv, bs = 70, 20, 4, 2, 16
+    rng = np.random.default_rng(77)
+    _, k, v, bt, _ = make_case(rng, 1, H, hkv, d, bs, dtype, [off + T])
+    q = rng.standard_normal((T, H, d)).astype(IO[dtype])
+    at = lambda j: (bt[0][j // bs], j % bs)
+    v[at(50)][0, 3], v[at(61)][1, d - 1], k[at(75)][0, 1], v[at(89)][1, 0] = np.inf, np.nan, np.nan, -np.inf
+    got = {}
+    for choice in (0, 1):
+        eng = _engine()
+        eng.set_decode_kernel(choice)
+        got[choice] = _prefill(eng, q, to_dev(k), to_dev(v), bt[0], T, layer(H, hkv, d, bs, dtype), True, off)
+    a, b = got[0].astype(np.float64), got[1].astype(np.float64)
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    assert np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+    assert np.isfinite(a[:30]).all() and not np.isfinite(a[30:, :, 3]).all()
+    fin = np.isfinite(b).all(axis=-1)
+    assert row_rel_err(a[fin], b[fin]) <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,d", [(0, 128), (0, 64), (1, 96), (0, 32), (0, 200)])
+def test_rows_code_object_bit_identical(dtype, d):
+    T, off, H, hkv, bs = 45, 700, 8, 4, 16
+    rng = np.random.default_rng(78)
+    _, k, v, bt, _ = make_case(rng, 1, H, hkv, d, bs, dtype, [off + T])
+    q = rng.standard_normal((T, H, d)).astype(IO[dtype])
+    got = []
+    for module in (False, True):
+        eng = _engine()
+        if module:
+            eng.load_module()
+            eng.set_module_strict(True)
+        got.append(_prefill(eng, q, to_dev(k), to_dev(v), bt[0], T, layer(H, hkv, d, bs, dtype), True, off))
+    assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))
+
+
+@pytest.mark.parametrize("dtype,H,hkv,d,bs,lens,window,part", [
+    (0, 8, 2, 128, 16, [0, 1, 15, 16, 17, 255, 256, 257], 0, 0),
+    (0, 32, 8, 64, 16, [5000, 33, 1290], 0, 0),         # several partitions and the reduce
+    (0, 6, 2, 80, 12, [700, 1, 64], 0, 48),             # G = 3, head size between tiles
+    (0, 20, 1, 36, 16, [100, 17], 0, 0),                # 20 heads a kv head: two slots, the second of 4
+    (0, 4, 4, 256, 8, [1500, 0, 300], 0, 0),
+    (0, 2, 2, 4, 1, [3, 40], 0, 0),
+    (1, 16, 16, 64, 16, [3000, 100, 17, 0], 0, 0),
+    (1, 8, 4, 128, 16, [2000, 500], 333, 0),
+    (1, 34, 2, 96, 32, [900, 31], 0, 0),                # 17 heads a kv head
+    (1, 8, 8, 256, 16, [260, 4], 0, 0),
+    (2, 8, 8, 128, 16, [1000, 1, 77], 0, 0),
+    (2, 12, 4, 64, 16, [2000, 48], 100, 32),
+    (2, 8, 4, 96, 4, [513, 2], 0, 0),
+])
+def test_decode_rows_parity(dtype, H, hkv, d, bs, lens, window, part):
+    import torch
+    rng = np.random.default_rng(1300 + d + len(lens))
+    eng = _engine()
+    q, k, v, bt, lens = make_case(rng, len(lens), H, hkv, d, bs, dtype, lens)
+    if dtype == 2:
+        kd, vd, ksd, vsd, k, v, ks, vs = build_fp8(eng, rng, k, v, bt, lens, hkv, d, bs)
+        ks, vs = ks.view(np.uint16), vs.view(np.uint16)
+    else:
+        kd, vd, ksd, vsd, ks, vs = to_dev(k), to_dev(v), None, None, None, None
+    eng.set_partition_tokens(part)
+    out = torch.full(q.shape, 7.0, dtype=torch.float32 if dtype == 0 else torch.float16, device="cuda")
+    eng.decode(to_dev(q), kd, vd, to_dev(bt), to_dev(lens), out, len(lens), bt.shape[1],
+               layer(H, hkv, d, bs, dtype, window), k_scale=ksd, v_scale=vsd)
+    ref = oracle.decode(dtype, q, k, v, bt, lens, H, window=window, k_scale=ks, v_scale=vs, n_threads=8)
+    o = to_host(out).astype(np.float64)
+    assert np.isnan(o[lens == 0]).all(), "a row without keys is 0/0"
+    assert row_rel_err(o[lens > 0], ref[lens > 0]) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,d", [(0, 128), (1, 64), (1, 96)])
+def test_decode_rows_read_nothing_past_a_row(dtype, d):
+    """NaN and Inf in the tail of a row's last block, and in its last visible key."""
+    import torch
+    H, hkv, bs = 8, 4, 16
+    rng = np.random.default_rng(79)
+    q, k, v, bt, lens = make_case(rng, 3, H, hkv, d, bs, dtype, [37, 300, 5])
+    for i, L in enumerate(lens):
+        b = bt[i][(L - 1) // bs]
+        k[b, L % bs:], v[b, L % bs:] = np.nan, np.inf
+    v[bt[1][299 // bs], 299 % bs, 0, 2] = np.inf
+    got = {}
+    for choice in (0, 1):
+        eng = _engine()
+        eng.set_decode_kernel(choice)
+        out = torch.empty(q.shape, dtype=torch.float32 if dtype == 0 else torch.float16, device="cuda")
+        eng.decode(to_dev(q), to_dev(k), to_dev(v), to_dev(bt), to_dev(lens), out, 3, bt.shape[1],
+                   layer(H, hkv, d, bs, dtype))
+        got[choice] = to_host(out).astype(np.float64)
+    a, b = got[0], got[1]
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    assert np.isinf(a).sum() == H // hkv
+    fin = np.isfinite(b).all(axis=-1)
+    assert row_rel_err(a[fin], b[fin]) <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,d,lens", [(0, 128, [700, 40]), (1, 64, [1000, 3]), (2, 96, [90, 300])])
+def test_decode_rows_code_object_bit_identical(dtype, d, lens):
+    import torch
+    H, hkv, bs = 8, 4, 16
+    rng = np.random.default_rng(80)
+    q, k, v, bt, lens = make_case(rng, len(lens), H, hkv, d, bs, dtype, lens)
+    ksd = vsd = None
+    if dtype == 2:
+        kd, vd, ksd, vsd, *_ = build_fp8(_engine(), rng, k, v, bt, lens, hkv, d, bs)
+    else:
+        kd, vd = to_dev(k), to_dev(v)
+    got = []
+    for module in (False, True):
+        eng = _engine()
+        if module:
+            eng.load_module()
+            eng.set_module_strict(True)
+        out = torch.empty(q.shape, dtype=torch.float32 if dtype == 0 else torch.float16, device="cuda")
+        eng.decode(to_dev(q), kd, vd, to_dev(bt), to_dev(lens), out, len(lens), bt.shape[1], layer(H, hkv, d, bs, dtype),
+                   k_scale=ksd, v_scale=vsd)
+        got.append(to_host(out))
+    assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))

@@ -4,6 +4,7 @@
 #include "rows_body.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace pam {
 
@@ -36,21 +37,46 @@ bool rows_supported(const AttnParams &p, int32_t dtype) {
 // query rows of a prefill block (kPrefillRowsRB)
 static int64_t block_rows(int32_t head_dim, int32_t dtype) { return dtype == kF32 && head_dim > 128 ? 16 : 32; }
 
-// Partition length of a prefill of p.rows rows over its keys: the workgroups of
-// the launch split the keys until there are about four per CU, in multiples of
-// 64 tokens (a tile for each of the four waves).
+// Partition length of a prefill of p.rows rows over its keys: the candidate whose
+// estimate is least.  Two workgroups fit a CU, two waves a SIMD.  The launch takes
+// the larger of its whole work over those places and its longest workgroup, half of
+// that again when the workgroups need several rounds, and partitions cost the
+// reduce.  The constants are fits to calls measured on gfx950 (µs, estimate /
+// measured: f32 8/8 d = 128, 777 tokens after 391 in partitions of 24 tiles 49 / 51,
+// of 12 65 / 61; 17 after 2000 in partitions of 4 17 / 17; 64 in one 11 / 8; f32 32/8
+// 2048 tokens in one 457 / 378, of 32 505 / 468).
 int32_t prefill_rows_part_tokens(const AttnParams &p, int32_t dtype, int32_t cus) {
+    constexpr double kStartUs = 8.0, kReduceUs = 4.0, kReduceGBs = 3000.0, kCyclesPerUs = 2400.0;
     const int64_t G = p.num_heads / p.num_kv_heads;
     const int64_t kv_len = (int64_t)p.q_offset + p.rows;
     const int64_t k_lo = p.window > 0 && kv_len > p.window ? (kv_len - p.window) / 16 * 16 : 0;
-    const int64_t R = block_rows(p.head_dim, dtype), nblocks = (p.rows * G + R - 1) / R;
-    const int64_t longest = kv_len - k_lo;
-    const int64_t shortest = p.causal ? std::max<int64_t>(0, p.q_offset + 1 - k_lo) : longest;
-    const int64_t tiles = nblocks * p.num_kv_heads * (longest + shortest) / 32;  // 16-key tiles, about
-    int64_t per = (tiles / (4 * (int64_t)(cus > 0 ? cus : 1)) + kRowsWaves - 1) / kRowsWaves * kRowsWaves;
-    if (per < kRowsWaves) per = kRowsWaves;
-    const int64_t whole = ((longest + 15) / 16 + 1) * 16;
-    return (int32_t)(per * 16 >= longest ? whole : per * 16);
+    const int64_t R = block_rows(p.head_dim, dtype), nblocks = (p.rows * G + R - 1) / R, nt = (p.head_dim + 31) / 32;
+    const int64_t longest = (kv_len - k_lo + 15) / 16;
+    const int64_t first = p.q_offset + (R + G - 1) / G;  // keys of the first block's last row
+    const int64_t shortest = p.causal ? std::max<int64_t>(0, (std::min(first, kv_len) - k_lo + 15) / 16) : longest;
+    // a tile's matrix cycles (f32: scores and outputs; else the outputs) and the rest of its work
+    const double tile_us = 1.4 * (R / 16) * (dtype == kF32 ? 512.0 : 280.0) * nt / kCyclesPerUs + 0.2;
+    const double tiles = 0.5 * (shortest + longest) * nblocks * p.num_kv_heads, places = 2.0 * (cus > 0 ? cus : 1);
+    double best = 1e300;
+    int64_t best_per = longest;
+    for (int64_t w = 1;; w = w < 8 ? w + 1 : w + w / 4) {  // tiles per wave
+        const int64_t per = w * kRowsWaves;
+        double groups = 0.0;
+        const int64_t samples = std::min<int64_t>(nblocks, 64);
+        for (int64_t i = 0; i < samples; i++) {
+            const int64_t t = samples > 1 ? shortest + (longest - shortest) * i / (samples - 1) : longest;
+            groups += (double)std::max<int64_t>(1, (t + per - 1) / per);
+        }
+        groups *= (double)nblocks / samples * p.num_kv_heads;
+        const double share = 2.0 * groups <= places ? 1.0 : 2.0;  // waves a SIMD
+        const double one = kStartUs + share * tile_us * (double)std::min(w, (longest + kRowsWaves - 1) / kRowsWaves);
+        double us = std::max(one, (groups * kStartUs + tiles / kRowsWaves * share * tile_us) / places);
+        if (groups > places) us += 0.5 * one;
+        if (per < longest) us += kReduceUs + 8.0 * groups * R * p.head_dim / (kReduceGBs * 1e3);
+        if (us < best) best = us, best_per = per;
+        if (per >= longest) break;
+    }
+    return (int32_t)(best_per >= longest ? (longest + 1) * 16 : best_per * 16);
 }
 
 #define PAM_ROWS_SWITCH(KERNEL)                                                                        \

@@ -188,17 +188,19 @@ struct RowTiles {
         for (int t = t0; t < t1; t += step) {
             const int kb = keys.key0 + 16 * t;
             const bool more = t + step < t1;
-            f32x4 s[RB];
+            f32x4 s[RB], s2[RB];  // f32: two chains of sums, which halves their rounding
 #pragma unroll
-            for (int b = 0; b < RB; b++) s[b] = (f32x4)0.0f;
+            for (int b = 0; b < RB; b++) s[b] = s2[b] = (f32x4)0.0f;
 #pragma unroll
             for (int c = 0; c < KC; c++) {
                 if constexpr (F32) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
+                    for (int e = 0; e < 4; e += 2)
 #pragma unroll
-                        for (int b = 0; b < RB; b++)
+                        for (int b = 0; b < RB; b++) {
                             s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[b][c][e], s[b], 0, 0, 0);
+                            s2[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e + 1], q[b][c][e + 1], s2[b], 0, 0, 0);
+                        }
                 } else {
                     f16x8 a;
                     if constexpr (sizeof(KV) == 1)
@@ -218,6 +220,9 @@ struct RowTiles {
                 issue_k(p, row_n, blk_n);
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (F32)
+#pragma unroll
+                for (int b = 0; b < RB; b++) s[b] += s2[b];
             // Online softmax.  The reference max of a row moves only when a score
             // passes it by 8, a factor of 2^8 (or the row has none yet): the probabilities
             // are f32, so their scale is free, and most tiles need no reduction across

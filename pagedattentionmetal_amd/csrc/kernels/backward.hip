@@ -16,6 +16,8 @@
 //   * bwd_keys_kernel: one wave per (key, kv head) recomputes P and dS over the
 //     rows of its head group and adds its dK/dV row to the pool once, summed in
 //     f32.
+// They serve what neither the f16 matrix kernels below nor backward_rows.hip takes:
+// head sizes that are not whole 8-element pieces (f16) and unaligned buffers.
 // Lanes hold dims lane + 64 t of the head (t < 4, d <= 256); dot products are
 // wave reductions, loads of a key or query row are 64 lanes over contiguous dims.
 #include <type_traits>
@@ -624,13 +626,23 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkv_mfma(BackwardParams
 
 constexpr int kBwdNB = 1;  // 32-row / 32-key blocks per wave (2 needs more than 512 registers)
 
+static int64_t table_entries(const BackwardParams &p) {
+    return p.block_size > 0 ? (int64_t)(p.seq_len - 1) / p.block_size - p.window_start / p.block_size + 1 : 0;
+}
+
+bool backward_mfma_supported(const BackwardParams &p, int32_t dtype) {
+    const int G = p.num_heads / p.num_kv_heads;
+    return dtype == kF16 && p.head_dim == 128 && (G & (G - 1)) == 0 && table_entries(p) <= kBwdBtCache;
+}
+
 hipError_t launch_backward(const BackwardParams &p, int32_t dtype, hipStream_t stream) {
     if (p.seq_len <= 0) return hipSuccess;
     if (p.head_dim > 64 * kBwdMaxDims || p.row_d == nullptr) return hipErrorInvalidValue;
+    if (p.row_blocks) return launch_backward_rows(p, dtype, stream);
     const dim3 rows(p.seq_len, p.num_heads), keys(p.seq_len - p.window_start, p.num_kv_heads);
     const int G = p.num_heads / p.num_kv_heads;
-    const int64_t nblk = p.block_size > 0 ? (int64_t)(p.seq_len - 1) / p.block_size - p.window_start / p.block_size + 1 : 0;
-    if (dtype == kF16 && p.head_dim == 128 && p.row_c != nullptr && (G & (G - 1)) == 0 && nblk <= kBwdBtCache) {
+    if (backward_mfma_supported(p, dtype) && p.row_c != nullptr) {
+        const int64_t nblk = table_entries(p);
         const int64_t qrows = (int64_t)p.seq_len * G;
         const int64_t nkeys = p.seq_len - p.window_start;
         const int per = 32 * kBwdWaves * kBwdNB, gs = __builtin_ctz((unsigned)G);

@@ -185,3 +185,20 @@ def test_decode_rows_code_object_bit_identical(dtype, d, lens):
                    k_scale=ksd, v_scale=vsd)
         got.append(to_host(out))
     assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))
+
+
+@pytest.mark.parametrize("dtype,T,H,hkv,d,bs,W", [
+    (0, 17, 3, 1, 32, 16, 0),        # G = 3, one row tile and one key past a tile
+    (0, 70, 6, 2, 80, 12, 33),       # head size between tiles, window inside a tile, odd blocks
+    (0, 260, 8, 1, 64, 16, 0),       # several shares per key block
+    (0, 100, 4, 2, 128, 16, 48),     # window at a tile boundary
+    (0, 40, 2, 2, 36, 1, 0),
+    (1, 33, 5, 1, 96, 16, 0),
+    (1, 300, 12, 4, 128, 16, 0),     # f16 d = 128 with a group that is no power of two
+    (1, 129, 32, 2, 64, 8, 100),
+    (1, 50, 4, 4, 256, 16, 0),
+    (1, 20, 2, 1, 40, 4, 0),
+])
+def test_backward_rows_parity(dtype, T, H, hkv, d, bs, W):
+    import test_gpu_backward
+    test_gpu_backward.test_backward_parity(dtype, T, H, hkv, d, bs, W)

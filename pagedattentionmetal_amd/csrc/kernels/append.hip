@@ -6,9 +6,9 @@
 // the input and the pool, so each thread moves one 16-byte piece of a row.
 //
 // kv_append_fp8 (kernels.metal:1876-1961): one workgroup per physical block the
-// append touches reduces max|k|, max|v| over this append's elements in that block
-// (all heads), derives the block's new half scale from the old one and quantizes
-// the new elements with it.  A deterministic block reduction replaces the
+// append touches and pool reduces max|k| or max|v| over this append's elements in
+// that block (all heads), derives the block's new half scale from the old one and
+// quantizes the new elements with it.  A deterministic block reduction replaces the
 // reference's scratch buffer + CAS atomics, and one launch replaces its two
 // synchronous passes.
 #include "append_body.h"
@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(AppendParams p, int64_t 
     append_body<CH>(p, chunks_per_row, total);
 }
 
-__global__ __launch_bounds__(256) void kv_append_fp8_kernel(AppendBatchParams p, int32_t first_lb,
+__global__ __launch_bounds__(kFp8Threads) void kv_append_fp8_kernel(AppendBatchParams p, int32_t first_lb,
                                                             int32_t single_offset) {
     append_fp8_body(p, first_lb, single_offset);
 }
@@ -57,11 +57,11 @@ hipError_t launch_append(const AppendParams &p, int32_t dtype, hipStream_t strea
         b.num_kv_heads = p.num_kv_heads;
         b.head_dim = p.head_dim;
         b.block_size = p.block_size;
-        const dim3 grid(last_lb - first_lb + 1);
+        const dim3 grid(last_lb - first_lb + 1, 2), block(kFp8Threads);  // K and V
         const int32_t off = p.token_offset;
         hipError_t e;
-        if (via_module(kt, kt ? kt->append_fp8 : nullptr, &e, grid, dim3(256), stream, b, first_lb, off)) return e;
-        hipLaunchKernelGGL(kv_append_fp8_kernel, grid, dim3(256), 0, stream, b, first_lb, off);
+        if (via_module(kt, kt ? kt->append_fp8 : nullptr, &e, grid, block, stream, b, first_lb, off)) return e;
+        hipLaunchKernelGGL(kv_append_fp8_kernel, grid, block, 0, stream, b, first_lb, off);
         return hipGetLastError();
     }
     const int64_t row_bytes = row_elems * (dtype == kF32 ? 4 : 2);
@@ -116,8 +116,9 @@ hipError_t launch_append_batch(const AppendBatchParams &p, int32_t dtype, hipStr
     if (p.num_work <= 0) return hipSuccess;
     const int32_t zero = 0;
     hipError_t e;
-    if (via_module(kt, kt ? kt->append_fp8 : nullptr, &e, dim3(p.num_work), dim3(256), stream, p, zero, zero)) return e;
-    hipLaunchKernelGGL(kv_append_fp8_kernel, dim3(p.num_work), dim3(256), 0, stream, p, 0, 0);
+    const dim3 grid(p.num_work, 2), block(kFp8Threads);
+    if (via_module(kt, kt ? kt->append_fp8 : nullptr, &e, grid, block, stream, p, zero, zero)) return e;
+    hipLaunchKernelGGL(kv_append_fp8_kernel, grid, block, 0, stream, p, 0, 0);
     return hipGetLastError();
 }
 

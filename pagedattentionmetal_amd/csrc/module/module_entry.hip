@@ -132,8 +132,8 @@ PAM_APPEND_ENTRY(pam_append_b2, uint16_t)
 PAM_APPEND_BATCH_ENTRY(pam_append_batch_b16, uint4)
 PAM_APPEND_BATCH_ENTRY(pam_append_batch_b4, uint32_t)
 PAM_APPEND_BATCH_ENTRY(pam_append_batch_b2, uint16_t)
-// FP8 quantize-on-append, one workgroup per touched block
-extern "C" __global__ __launch_bounds__(256) void pam_append_fp8(AppendBatchParams p, int32_t first_lb,
+// FP8 quantize-on-append, one workgroup per touched block and pool
+extern "C" __global__ __launch_bounds__(kFp8Threads) void pam_append_fp8(AppendBatchParams p, int32_t first_lb,
                                                                  int32_t single_offset) {
     append_fp8_body(p, first_lb, single_offset);
 }

@@ -486,14 +486,16 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkv_mfma(BackwardParams
         }
     }
     const float sl2 = p.scale * kLog2e;
-    const int NT = (rows + 31) / 32;
+    // this workgroup's share of the row tiles: [tb, tb + NT) of all of them
+    const int all = (rows + 31) / 32, per = (all + p.shares - 1) / p.shares, tb = (int)blockIdx.z * per;
+    const int NT = all - tb < per ? all - tb : per;
     auto head_row = [&](int r) -> int64_t {
         r = r < rows ? r : rows - 1;
         return (int64_t)(r >> group_shift) * H + kvh * G + (r & (G - 1));
     };
     auto issue = [&](int t) {
         const int w = t % R;
-        t = t < NT ? t : NT - 1;
+        t = tb + (t < NT ? t : NT - 1);
         tile_dma(q_lds[w], wave, lane, [&](int Rw) { return Q + head_row(t * 32 + Rw) * 128; });
         tile_dma(g_lds[w], wave, lane, [&](int Rw) { return dO + head_row(t * 32 + Rw) * 128; });
         const float *src = (wave & 1) ? p.row_d : p.row_c;
@@ -501,9 +503,9 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkv_mfma(BackwardParams
         if (lane < 32) lds_dma4(src + head_row(t * 32 + lane), dst);
     };
     // rows of the last tile past the end: c = +inf (P = 0); its loads are done
-    const int tail = rows - 32 * (NT - 1);
+    const int tail = rows - 32 * (all - 1);
     auto patch_tail = [&](int t) {
-        if (t == NT - 1 && tail < 32 && tid >= tail && tid < 32) c_lds[t % R][tid] = INFINITY;
+        if (tb + t == all - 1 && tail < 32 && tid >= tail && tid < 32) c_lds[t % R][tid] = INFINITY;
     };
     const TrAddr ta = tr_addr(lane);
     bw_f32x16 dk[4], dv[4];  // in AGPRs (mfma_agpr)
@@ -604,7 +606,20 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkv_mfma(BackwardParams
     for (int dt = 0; dt < 4; dt++) asm volatile("" : "+a"(dk[dt]), "+a"(dv[dt]));
     ring_barrier<0>();  // the loads issued past the last tile
     const float fk = p.scale / kBwdPScale, fv = 1.0f / kBwdPScale;
-    if (key < T) {
+    if (key < T && p.shares > 1) {
+        // f32 partials, summed into the pools by bwd_dkv_sum
+        const int64_t row = (int64_t)(key - ws) * p.num_kv_heads + kvh, n = (int64_t)(T - ws) * p.num_kv_heads;
+        float *dkr = p.partial + (2 * (int64_t)blockIdx.z * n + row) * 128 + 4 * h, *dvr = dkr + n * 128;
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                *reinterpret_cast<float4 *>(dkr + 32 * dt + 8 * q) = make_float4(
+                    dk[dt][4 * q] * fk, dk[dt][4 * q + 1] * fk, dk[dt][4 * q + 2] * fk, dk[dt][4 * q + 3] * fk);
+                *reinterpret_cast<float4 *>(dvr + 32 * dt + 8 * q) = make_float4(
+                    dv[dt][4 * q] * fv, dv[dt][4 * q + 1] * fv, dv[dt][4 * q + 2] * fv, dv[dt][4 * q + 3] * fv);
+            }
+    } else if (key < T) {
         f16 *dkr = const_cast<f16 *>(pool_row(static_cast<const f16 *>(p.d_k_pool), p, key, kvh)) + 4 * h;
         f16 *dvr = const_cast<f16 *>(pool_row(static_cast<const f16 *>(p.d_v_pool), p, key, kvh)) + 4 * h;
 #pragma unroll
@@ -635,6 +650,28 @@ bool backward_mfma_supported(const BackwardParams &p, int32_t dtype) {
     return dtype == kF16 && p.head_dim == 128 && (G & (G - 1)) == 0 && table_entries(p) <= kBwdBtCache;
 }
 
+// Shares of the query rows of a bwd_dkv_mfma key block.  A workgroup fills a CU, so
+// few key blocks leave CUs idle: the count whose estimate is least, of rounds of
+// workgroups (a row tile takes 1.04 µs, a workgroup's start and end 6) and, from two
+// shares on, of the partials written and summed.  Measured on gfx950 (µs, one share
+// -> the count chosen; the whole backward): 32/8 heads T = 2048 444 -> 359 (dK / dV
+// 267 -> 173 and the sum 9), T = 300 79 -> 53; 32/2 T = 996 558 -> 142.
+int32_t backward_mfma_shares(const BackwardParams &p, int32_t cus) {
+    const int64_t keys = p.seq_len - p.window_start, per = 32 * kBwdWaves;
+    const int64_t blocks = (keys + per - 1) / per * p.num_kv_heads;
+    const int64_t tiles = ((int64_t)p.seq_len * (p.num_heads / p.num_kv_heads) + 31) / 32;
+    double best = 1e300;
+    int32_t best_s = 1;
+    for (int64_t s = 1; s <= 32 && s <= tiles; s++) {
+        const int64_t rounds = (blocks * s + cus - 1) / (cus > 0 ? cus : 1), each = (tiles + s - 1) / s;
+        if ((tiles + each - 1) / each != s) continue;  // every share has a tile
+        double us = (double)rounds * (each * 1.04 + 6.0);
+        if (s > 1) us += 5.0 + (double)(2 * s + 2) * keys * p.num_kv_heads * 128 * 4 / 3.5e6;
+        if (us < best) best = us, best_s = (int32_t)s;
+    }
+    return best_s;
+}
+
 hipError_t launch_backward(const BackwardParams &p, int32_t dtype, hipStream_t stream) {
     if (p.seq_len <= 0) return hipSuccess;
     if (p.head_dim > 64 * kBwdMaxDims || p.row_d == nullptr) return hipErrorInvalidValue;
@@ -651,9 +688,13 @@ hipError_t launch_backward(const BackwardParams &p, int32_t dtype, hipStream_t s
             hipLaunchKernelGGL((bwd_dq_mfma<kBwdNB, kBwdBtCacheSmall>), dq_grid, dim3(64 * kBwdWaves), 0, stream, p, gs);
         else
             hipLaunchKernelGGL((bwd_dq_mfma<kBwdNB, kBwdBtCache>), dq_grid, dim3(64 * kBwdWaves), 0, stream, p, gs);
-        if (nkeys > 0)
-            hipLaunchKernelGGL(bwd_dkv_mfma<kBwdNB>, dim3((unsigned)((nkeys + per - 1) / per), p.num_kv_heads),
+        if (p.shares < 1 || (p.shares > 1 && p.partial == nullptr)) return hipErrorInvalidValue;
+        if (nkeys > 0) {
+            hipLaunchKernelGGL(bwd_dkv_mfma<kBwdNB>,
+                               dim3((unsigned)((nkeys + per - 1) / per), p.num_kv_heads, (unsigned)p.shares),
                                dim3(64 * kBwdWaves), 0, stream, p, gs);
+            if (p.shares > 1) return launch_backward_sum(p, dtype, stream);
+        }
         return hipGetLastError();
     }
     if (dtype == kF32) {

@@ -438,6 +438,16 @@ int32_t backward_rows_shares(const BackwardParams &p, int32_t dtype, int32_t cus
     return dtype == kF32 ? shares_of<float>(p, cus) : shares_of<f16>(p, cus);
 }
 
+hipError_t launch_backward_sum(const BackwardParams &p, int32_t dtype, hipStream_t stream) {
+    const int64_t n = (int64_t)(p.seq_len - p.window_start) * p.num_kv_heads * (p.head_dim / 4);
+    const dim3 grid((unsigned)((n + 255) / 256), 2);
+    if (dtype == kF32)
+        hipLaunchKernelGGL(bwd_dkv_sum<float>, grid, dim3(256), 0, stream, p);
+    else
+        hipLaunchKernelGGL(bwd_dkv_sum<f16>, grid, dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
 template <typename T>
 static hipError_t launch_type(const BackwardParams &p, hipStream_t stream) {
     return with_shape<T>(p, [&](auto shape) {
@@ -451,9 +461,7 @@ static hipError_t launch_type(const BackwardParams &p, hipStream_t stream) {
             hipLaunchKernelGGL((bwd_dkv_rows<T, S>),
                                dim3((unsigned)((keys + kspan - 1) / kspan * p.num_kv_heads), (unsigned)p.shares), block, 0,
                                stream, p);
-            const int64_t n = keys * p.num_kv_heads * (p.head_dim / 4);
-            if (p.shares > 1)
-                hipLaunchKernelGGL(bwd_dkv_sum<T>, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, stream, p);
+            if (p.shares > 1) return launch_backward_sum(p, sizeof(T) == 4 ? kF32 : kF16, stream);
         }
         return hipGetLastError();
     });

@@ -245,19 +245,24 @@ struct BackwardParams {
     int32_t num_heads, num_kv_heads, head_dim, block_size;
     float scale;  // 1 / sqrt(head_dim)
     // row-block form (backward_rows.hip): row_d then holds the rows' {m, 1 / l, D,
-    // 0} ([Hkv][rows of the group] float4), and `shares` > 1 workgroups per key
-    // block leave their dK / dV in `partial` ([shares][2][keys][Hkv][d] floats)
-    int32_t row_blocks, shares;
+    // 0} ([Hkv][rows of the group] float4)
+    int32_t row_blocks;
+    // matrix forms: `shares` > 1 workgroups per key block leave their dK / dV in
+    // `partial` ([shares][2][keys][Hkv][d] floats)
+    int32_t shares;
     float *partial;
     const void *zero_page;
 };
 hipError_t launch_backward(const BackwardParams &p, int32_t dtype, hipStream_t stream);
 // f16, d = 128, power-of-two groups: the f16 matrix kernels
 bool backward_mfma_supported(const BackwardParams &p, int32_t dtype);
+int32_t backward_mfma_shares(const BackwardParams &p, int32_t cus);
 // the f32-probability matrix kernels (backward_rows.hip)
 bool backward_rows_supported(const BackwardParams &p, int32_t dtype);
 int32_t backward_rows_shares(const BackwardParams &p, int32_t dtype, int32_t cus);
 hipError_t launch_backward_rows(const BackwardParams &p, int32_t dtype, hipStream_t stream);
+// the shares' partials, summed in order, into the gradient pools
+hipError_t launch_backward_sum(const BackwardParams &p, int32_t dtype, hipStream_t stream);
 
 // Exhaustive codec entry points (used by the codec tests through the C ABI).
 hipError_t launch_fp8_quantize(const uint16_t *values, const uint16_t *scales, uint8_t *out, int64_t n,

@@ -1306,18 +1306,22 @@ void Context::backward(const pam_backward_request &r) {
     const int64_t row_heads = (int64_t)r.seq_len * l.num_heads;
     // two floats per (row, head); the row-block form keeps four, then its partials
     int64_t floats = row_heads * 2;
-    if (!backward_mfma_supported(p, l.data_type) && backward_rows_supported(p, l.data_type)) {
+    p.shares = 1;
+    if (backward_mfma_supported(p, l.data_type)) {
+        p.shares = backward_mfma_shares(p, cus_);
+    } else if (backward_rows_supported(p, l.data_type)) {
         p.row_blocks = 1;
         p.shares = backward_rows_shares(p, l.data_type, cus_);
         floats = row_heads * 4;
-        if (p.shares > 1)
-            floats += (int64_t)p.shares * 2 * (r.seq_len - p.window_start) * l.num_kv_heads * l.head_dim;
     }
+    const int64_t partial = (floats + 3) / 4 * 4;  // 16-byte aligned
+    if (p.shares > 1)
+        floats = partial + (int64_t)p.shares * 2 * (r.seq_len - p.window_start) * l.num_kv_heads * l.head_dim;
     const int64_t tmp = floats * 4;
     reserve_workspace((size_t)tmp);
     p.row_d = static_cast<float *>(workspace_.ptr);
     p.row_c = p.row_d + row_heads;
-    p.partial = p.row_d + row_heads * 4;
+    p.partial = p.row_d + partial;
     with_retry("backward", [&] {
         mark(ev0_);
         check_launch([&] { return launch_backward(p, l.data_type, stream()); }, "backward");

@@ -29,11 +29,11 @@
 
 namespace pam {
 
-template <typename KV, int HD, int BLK>
+template <typename KV, int HD, int BLK, bool FL>
 __global__ __launch_bounds__(64 * kMfmaWaves, (MfmaShape<KV, HD>::OCC)) void attn_mfma_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) char smem[MfmaShape<KV, HD>::kSmemBytes];
     __shared__ float sm_ml[kMfmaWaves][16][2];
-    mfma_item<KV, HD, BLK>(p, blockIdx.z, blockIdx.x, blockIdx.y, smem, sm_ml);
+    mfma_item<KV, HD, BLK, FL>(p, blockIdx.z, blockIdx.x, blockIdx.y, smem, sm_ml);
 }
 
 // The kernel (the fat binary's entry); streamk_body also backs the named
@@ -58,9 +58,9 @@ __global__ __launch_bounds__(64 * kValuWgMaxParts) void attn_valu_wg_kernel(Attn
     valu_body<KV, QT, NH, true>(p, lanes_per_row, wg_lds);
 }
 
-template <typename QT>
+template <typename QT, bool FL>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(AttnParams p) {
-    reduce_body<QT>(p);
+    reduce_body<QT, FL>(p);
 }
 
 // ------------------------------------------------------------------ launchers
@@ -125,10 +125,13 @@ static hipError_t launch_mfma_blk(const AttnParams &p, hipStream_t stream, const
     }
     const dim3 grid(p.max_parts, p.num_kv_heads, p.rows);
     hipError_t me;
-    if (via_module(kt, kt && HD == 128 && BLK == kBlkTile ? kt->mfma_wg[sizeof(KV) == 1] : nullptr, &me, grid, block,
-                   stream, p))
+    if (via_module(kt, kt && HD == 128 && BLK == kBlkTile ? kt->mfma_wg[sizeof(KV) == 1][p.fused_layers > 1] : nullptr,
+                   &me, grid, block, stream, p))
         return me;
-    hipLaunchKernelGGL((attn_mfma_kernel<KV, HD, BLK>), grid, block, 0, stream, p);
+    if (p.fused_layers > 1)
+        hipLaunchKernelGGL((attn_mfma_kernel<KV, HD, BLK, true>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((attn_mfma_kernel<KV, HD, BLK, false>), grid, block, 0, stream, p);
     return hipGetLastError();
 }
 
@@ -217,13 +220,16 @@ static hipError_t launch_valu(const AttnParams &p, hipStream_t stream, const Ker
 }
 
 hipError_t launch_reduce(const AttnParams &p, int32_t dtype, hipStream_t stream, const KernelTable *kt) {
-    const dim3 grid((p.num_heads + 3) / 4, p.rows);
+    const bool fl = p.fused_layers > 1;  // f16 outputs only
+    const dim3 grid((p.num_heads * (fl ? p.fused_layers : 1) + 3) / 4, p.rows);
     hipError_t e;
-    if (via_module(kt, kt ? kt->reduce[dtype != kF32] : nullptr, &e, grid, dim3(256), stream, p)) return e;
-    if (dtype == kF32)
-        hipLaunchKernelGGL((attn_reduce_kernel<float>), grid, dim3(256), 0, stream, p);
+    if (via_module(kt, kt ? kt->reduce[fl ? 2 : dtype != kF32] : nullptr, &e, grid, dim3(256), stream, p)) return e;
+    if (fl)
+        hipLaunchKernelGGL((attn_reduce_kernel<f16, true>), grid, dim3(256), 0, stream, p);
+    else if (dtype == kF32)
+        hipLaunchKernelGGL((attn_reduce_kernel<float, false>), grid, dim3(256), 0, stream, p);
     else
-        hipLaunchKernelGGL((attn_reduce_kernel<f16>), grid, dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((attn_reduce_kernel<f16, false>), grid, dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -436,24 +436,22 @@ __device__ __forceinline__ void mfma_core(const AttnParams &p, const RowCtx &c, 
 // share of the partition's tiles; the waves merge their softmax states in LDS
 // and write the output (one partition) or the partial for the reduce kernel.
 // Returns uniformly across the workgroup.
-template <typename KV, int HD, int BLK>
+template <typename KV, int HD, int BLK, bool FL = false>
 __device__ __forceinline__ void mfma_item(const AttnParams &p, int r, int part, int kvh, char *smem,
                                           float (*sm_ml)[16][2]) {
     using S = MfmaShape<KV, HD>;
     constexpr int NO = S::NO, NW = S::NW, WT = S::WT;
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63, row = lane & 15, grp = lane >> 4;
-    const int H = p.num_heads;
-    const int G = H / p.num_kv_heads;
+    const int G = slot_group<FL>(p), H = G * p.num_kv_heads;  // query-head slots
     const RowCtx c = row_ctx(p, r);
     const PartRange wg = part_range(c, part, p.part_tokens);
     if (part >= (wg.nparts > 1 ? wg.nparts : 1)) return;
     const bool head_ok = row < G;
-    f16 *out = static_cast<f16 *>(p.out);
     if (wg.nparts == 0) {
         // no keys: 0/0 as in the reference's m/l bookkeeping
         for (int idx = threadIdx.x; idx < G * HD; idx += 64 * NW)
-            out[(c.out_row * H + kvh * G) * (int64_t)HD + idx] = (f16)__builtin_nanf("");
+            out_head<FL, f16>(p, c.out_row, kvh, idx / HD)[idx % HD] = (f16)__builtin_nanf("");
         return;
     }
     // this wave's contiguous share of the workgroup's tiles (possibly empty)
@@ -465,7 +463,7 @@ __device__ __forceinline__ void mfma_item(const AttnParams &p, int r, int part, 
     }
     float m_run, l_run;
     f32x4 o[NO];
-    mfma_core<KV, HD, BLK, false>(p, c, kvh, pr, reinterpret_cast<f16 *>(smem) + wave * WT, m_run, l_run, o);
+    mfma_core<KV, HD, BLK, FL>(p, c, kvh, pr, reinterpret_cast<f16 *>(smem) + wave * WT, m_run, l_run, o);
     float l_tot = l_run + shfl_xor(l_run, 16);
     l_tot += shfl_xor(l_tot, 32);
 
@@ -499,15 +497,14 @@ __device__ __forceinline__ void mfma_item(const AttnParams &p, int r, int part, 
 #pragma unroll
             for (int q = 0; q < 4; q++) acc[q] += wt * v[q];
         }
-        const int hq = kvh * G + hh;
         if (wg.nparts == 1) {
             const float inv = 1.0f / den;
             f16x4 v;
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = (f16)(acc[q] * inv);
-            *reinterpret_cast<f16x4 *>(out + (c.out_row * H + hq) * (int64_t)HD + d) = v;
+            *reinterpret_cast<f16x4 *>(out_head<FL, f16>(p, c.out_row, kvh, hh) + d) = v;
         } else {
-            const int64_t slot = ((int64_t)r * H + hq) * p.max_parts + part;
+            const int64_t slot = ((int64_t)r * H + kvh * G + hh) * p.max_parts + part;
             *reinterpret_cast<f32x4 *>(p.part_o + slot * HD + d) = (f32x4){acc[0], acc[1], acc[2], acc[3]};
             if (d == 0) {
                 p.part_ml[slot * 2 + 0] = M;

@@ -75,8 +75,8 @@ struct AttnParams {
     // decode over layers sharing one pool (decodeLayers): the heads of
     // fused_layers layers share every K/V tile, so query-head slot v of a kv
     // head is head v % G of layer v / G, read from layer_q[v / G] and written to
-    // layer_out[v / G].  fused_layers <= 1: p.q / p.out only.  Stream-K MFMA
-    // decode only (G * fused_layers <= 16).
+    // layer_out[v / G].  fused_layers <= 1: p.q / p.out only.  MFMA decode only
+    // (G * fused_layers <= 16).
     int32_t fused_layers;
     const void *layer_q[kMaxFusedLayers];
     void *layer_out[kMaxFusedLayers];
@@ -98,14 +98,14 @@ struct AttnParams {
 // kernel body.
 struct KernelTable {
     hipFunction_t streamk[2][2];  // decode stream-K, d = 128, blocks >= 16: [f16, e4m3][one layer, fused layers]
-    hipFunction_t mfma_wg[2];     // decode, workgroup form (rows > 2048), d = 128, blocks >= 16: f16, e4m3
+    hipFunction_t mfma_wg[2][2];  // decode, workgroup form, d = 128, blocks >= 16: [f16, e4m3][one layer, fused layers]
     hipFunction_t prefill[2][3];  // dense prefill, [d = 128, d = 64][f16, f16 with fused append, e4m3]
     hipFunction_t mixed[2];       // one-launch mixed step: f16, e4m3
     hipFunction_t valu[3][4];     // VALU rows: [f32, f16, e4m3 KV][1, 2, 4, 8 heads per wave]
     hipFunction_t valu_wg[3][2];  // their workgroup form: [KV][1, 2 heads per wave]
     // row blocks (rows.hip): [f32, f16, e4m3 KV][head size up to 32, 64, 96, 128, 256]
     hipFunction_t prefill_rows[3][5], decode_rows[3][5];
-    hipFunction_t reduce[2];      // split-context reduce: f32, f16 outputs
+    hipFunction_t reduce[3];      // split-context reduce: f32, f16 outputs, f16 of fused layers
     hipFunction_t append[3];      // append copy in 16-, 4- or 2-byte pieces
     hipFunction_t append_batch[3];
     hipFunction_t append_fp8;     // FP8 quantize-on-append (single sequence and batched)

@@ -346,16 +346,17 @@ __device__ __forceinline__ void valu_body(const AttnParams &p, int lanes_per_row
 // partials' maxima and sums are reduced across lanes (one partition per lane),
 // then lane groups of HD/4 lanes each accumulate a share of the partitions'
 // weighted outputs and the groups are summed with shuffles.
-template <typename QT>
+template <typename QT, bool FL = false>
 __device__ __forceinline__ void reduce_body(const AttnParams &p) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = blockIdx.y, h = blockIdx.x * 4 + wave;
-    if (h >= p.num_heads) return;
+    const int G = slot_group<FL>(p), H = G * p.num_kv_heads;  // query-head slots
+    if (h >= H) return;
     const RowCtx c = row_ctx(p, r);
     const PartRange pr = part_range(c, 0, p.part_tokens);
     const int np = pr.nparts;
     if (np <= 1) return;
-    const int HD = p.head_dim, H = p.num_heads;
+    const int HD = p.head_dim;
     const int64_t base = ((int64_t)r * H + h) * p.max_parts;
     // one pass over (m, l): each lane folds its partitions, then the lanes merge
     float Ml = -INFINITY, dl = 0.0f;
@@ -389,7 +390,7 @@ __device__ __forceinline__ void reduce_body(const AttnParams &p) {
         const float inv = 1.0f / den;
 #pragma unroll
         for (int e = 0; e < 4; e++) a[e] *= inv;
-        store4<QT>(static_cast<QT *>(p.out) + (c.out_row * H + h) * (int64_t)HD + d0, a);
+        store4<QT>(out_head<FL, QT>(p, c.out_row, h / G, h % G) + d0, a);
     }
 }
 

@@ -23,12 +23,12 @@ namespace pam {
         AttnParams p) {                                                                                \
         streamk_body<KV, HD, BLK, FL>(p, blockIdx.x, gridDim.x);                                     \
     }
-#define PAM_WG_ENTRY(NAME, KV)                                                                        \
+#define PAM_WG_ENTRY(NAME, KV, FL)                                                                    \
     extern "C" __global__ __launch_bounds__(64 * kMfmaWaves, (MfmaShape<KV, 128>::OCC)) void NAME( \
         AttnParams p) {                                                                                \
         __shared__ __attribute__((aligned(16))) char smem[MfmaShape<KV, 128>::kSmemBytes];           \
         __shared__ float sm_ml[kMfmaWaves][16][2];                                                    \
-        mfma_item<KV, 128, kBlkTile>(p, blockIdx.z, blockIdx.x, blockIdx.y, smem, sm_ml);             \
+        mfma_item<KV, 128, kBlkTile, FL>(p, blockIdx.z, blockIdx.x, blockIdx.y, smem, sm_ml);         \
     }
 #define PAM_PREFILL_ENTRY(NAME, HD, FUSED, KV)                                               \
     extern "C" __global__ __launch_bounds__(64 * kPrefillWaves, 1) void NAME(AttnParams p) { \
@@ -72,9 +72,11 @@ PAM_STREAMK_ENTRY(pam_decode_streamk_e4m3_d128, uint8_t, 128, kBlkTile, false)
 // decodeLayers: the heads of several layers per K/V tile
 PAM_STREAMK_ENTRY(pam_decode_layers_streamk_f16_d128, f16, 128, kBlkTile, true)
 PAM_STREAMK_ENTRY(pam_decode_layers_streamk_e4m3_d128, uint8_t, 128, kBlkTile, true)
-// decode, workgroup form (more rows than the stream-K form takes)
-PAM_WG_ENTRY(pam_decode_wg_f16_d128, f16)
-PAM_WG_ENTRY(pam_decode_wg_e4m3_d128, uint8_t)
+// decode, workgroup form (small calls, and more rows than the stream-K form takes)
+PAM_WG_ENTRY(pam_decode_wg_f16_d128, f16, false)
+PAM_WG_ENTRY(pam_decode_wg_e4m3_d128, uint8_t, false)
+PAM_WG_ENTRY(pam_decode_layers_wg_f16_d128, f16, true)
+PAM_WG_ENTRY(pam_decode_layers_wg_e4m3_d128, uint8_t, true)
 // VALU rows (f32 KV, groups below 4): KV type and query heads per wave
 PAM_VALU_ENTRY(pam_decode_valu_f32_h1, float, float, 1)
 PAM_VALU_ENTRY(pam_decode_valu_f32_h2, float, float, 2)
@@ -99,6 +101,7 @@ PAM_VALU_WG_ENTRY(pam_decode_valu_wg_e4m3_h2, uint8_t, f16, 2)
 // split-context reduce, by output type
 extern "C" __global__ __launch_bounds__(256) void pam_reduce_f32(AttnParams p) { reduce_body<float>(p); }
 extern "C" __global__ __launch_bounds__(256) void pam_reduce_f16(AttnParams p) { reduce_body<f16>(p); }
+extern "C" __global__ __launch_bounds__(256) void pam_reduce_layers_f16(AttnParams p) { reduce_body<f16, true>(p); }
 // dense chunked prefill, d = 128 and d = 64
 PAM_PREFILL_ENTRY(pam_prefill_f16_d128, 128, false, f16)
 PAM_PREFILL_ENTRY(pam_prefill_fused_f16_d128, 128, true, f16)

@@ -338,6 +338,49 @@ static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles)
            (p.head_dim > 64 || (int64_t)p.rows * p.num_heads >= 512);
 }
 
+// Partition length, in 16-token tiles, of an MFMA decode that runs as partitions
+// (attn_mfma_kernel, merged by the reduce) rather than as stream-K; 0: stream-K.
+// The stream-K kernel streams a large call at the memory's rate, but a call pays
+// about 20 µs for finding its units' rows and merging them behind the stream.  A
+// small call's partitions are independent workgroups: about one per CU, cut to 128
+// tokens or more, and to one partition up to 512 tokens (256 at d = 256), where the
+// reduce would cost more than the shorter rows save.  Small: 150 MB of K and V by the
+// table's length (with rows of a byte a dim or two; a wider row is a workgroup's work
+// but no more of its latency).  Measured on gfx950 (µs per call, stream-K /
+// partitions, rows of L / 8 to L tokens, 32/8 heads): f16 d = 128: 1 row L = 2000 18.1
+// / 11.8, 8 rows L = 500 24.2 / 11.3, L = 2000 22.9 / 17.5, 32 rows L = 200 29.3 / 9.3,
+// L = 1000 28.0 / 20.1, 64 rows L = 500 30.7 / 21.9, L = 1000 33.6 / 38.0, 128 rows L =
+// 200 34.1 / 23.6, L = 500 37.6 / 39.6, 16 rows L = 4000 34.2 / 39.0; e4m3 d = 128: 32
+// rows L = 1000 26.0 / 17.4, L = 4000 37.8 / 45.8, 128 rows L = 500 33.2 / 25.2, L =
+// 1000 40.1 / 41.4; f16 d = 64: 32 rows L = 1000 21.3 / 12.6; d = 256 (64/8): 32 rows
+// L = 1000 47.5 / 34.8, 128 rows L = 500 77.5 / 75.1, 256 rows L = 200 74.1 / 93.8.
+static int64_t mfma_part_tiles(int64_t pairs, int64_t max_tiles, int32_t head_dim, int32_t dtype, int32_t cus) {
+    if (max_tiles <= 0) return 0;
+    const int64_t row_bytes = std::min<int64_t>(2 * (int64_t)head_dim * elem_bytes(dtype), 512);
+    if (pairs * max_tiles * 16 * row_bytes <= 150000000) {
+        if (max_tiles <= (head_dim > 128 ? 16 : 32)) return max_tiles;
+        int64_t t = 8;
+        while (t < 32 && t * 32 < max_tiles) t *= 2;  // at most 32 partials to merge, up to 512 tokens
+        // e4m3, whose workgroups wait on their widening more than on memory, up to
+        // 1.5 a CU (3 rows L = 4000: 14.6 at 256 tokens, 16.5 at 512; f16 21.1, 18.3)
+        const int64_t most = dtype == kFP8 ? cus + cus / 2 : cus + cus / 4;
+        while (t < max_tiles && pairs * ceil_div(max_tiles, t) > most) t *= 2;
+        t = std::min(t, max_tiles);
+        // a workgroup's own stream must stay short: 1024 tokens, or 2048 where
+        // that is the whole row or there are few pairs
+        if (t <= 64 || (t <= 128 && (t == max_tiles || pairs <= 64))) return t;
+    }
+    // few pairs of long rows: units of one pair would merge one batch after
+    // another (µs per call, stream-K / 256-token partitions: 1 row 64K tokens 87.6 /
+    // 65.9, 2 rows 16K 49.2 / 44.0; 2 rows 64K 99.1 / 103.2)
+    if (pairs <= 8 || (pairs <= 16 && max_tiles <= 2048)) {
+        int64_t t = 64;
+        while (t > 16 && pairs * ceil_div(max_tiles, t) < 3 * (int64_t)cus) t /= 2;
+        return t;
+    }
+    return 0;
+}
+
 // Split-context set-up of a row launch (p.rows and the shape already filled).
 // The MFMA kernel runs in its stream-K form when the rows fit it: partial slots
 // in the workspace plus the counters, no reduce kernel.  Otherwise rows are cut
@@ -358,26 +401,40 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
                         "-byte scratch.");
     };
     // a partition length set through pam_set_partition_tokens selects the
-    // partitioned form.  So do few (row, kv head) pairs with long contexts:
-    // there the stream-K form's last unit of a pair merges many partials one
-    // batch after another, where fixed partitions, split over a workgroup's
-    // waves and merged by the reduce kernel, keep every step short.  Measured
-    // on gfx950 (32/8 heads, f16, µs per call, stream-K -> partitions):
-    //   1 row:  2K tokens 20.8 -> 14.5, 4K 23.8 -> 15.1, 16K 43.5 -> 27.2, 64K 87.6 -> 65.9
-    //   2 rows: 4K 24.3 -> 16.3, 16K 49.2 -> 44.0, 64K 99.1 -> 103.2
-    //   4 rows: 2K 22.1 -> 16.3, 4K 27.6 -> 25.1, 16K 56.6 -> 58.9, 64K 168 -> 201
-    const int64_t pairs = (int64_t)p.rows * p.num_kv_heads;
-    const bool few_pairs = p.fused_layers <= 1 && max_tiles >= 128 &&
-                           (pairs <= 8 || (pairs <= 16 && max_tiles <= 2048) || (pairs <= 32 && max_tiles <= 256));
-    if (use_mfma && part_tokens_override == 0 && !few_pairs && mfma_streamk_plan(p, dtype, &slots, &counters)) {
+    // partitioned form, and so do small calls (mfma_part_tiles)
+    const int64_t pairs = (int64_t)p.rows * p.num_kv_heads, layers = p.fused_layers > 1 ? p.fused_layers : 1;
+    if (fixed) {
+        // The limits of the allocation-free decode are those of the stream-K and
+        // VALU forms (and of partitions for few pairs), whichever form then runs: a
+        // request is refused by its shape alone, not by how fast a form is.
+        const bool few = max_tiles >= 128 && (pairs <= 8 || (pairs <= 16 && max_tiles <= 2048) ||
+                                              (pairs <= 32 && max_tiles <= 256));
+        int64_t bytes = 0, count = 0;
+        if (use_mfma && part_tokens_override == 0 && !few && mfma_streamk_plan(p, dtype, &slots, &counters)) {
+            bytes = slots * ((int64_t)p.head_dim + 2) * 4;
+            count = counters;
+        } else {
+            const int64_t parts = max_tiles > 0 ? ceil_div(max_tiles, choose_part_tokens(waves, max_tiles, use_mfma) / 16) : 1;
+            if (parts > 1 && (use_mfma || p.heads_per_wave > 2 || parts > kValuWgMaxParts)) {
+                bytes = (int64_t)p.rows * p.num_heads * parts * ((int64_t)p.head_dim + 2) * 4;
+                count = use_mfma ? 0 : (int64_t)p.rows * (p.num_heads / p.heads_per_wave);
+            }
+        }
+        if (bytes > fixed_parts) throw too_big("split-context partials", bytes, fixed_parts);
+        if (count * 8 > (int64_t)kNoAllocCounterBytes)
+            throw too_big("merge counters", count * 8, (int64_t)kNoAllocCounterBytes);
+    }
+    int64_t part_tiles =
+        use_mfma && part_tokens_override == 0 ? mfma_part_tiles(pairs, max_tiles, p.head_dim, dtype, cus_) : 0;
+    if (fixed && part_tiles > 0 && part_tiles < max_tiles &&
+        p.rows * (int64_t)p.num_heads * ceil_div(max_tiles, part_tiles) * (p.head_dim + 2) * 4 > fixed_parts)
+        part_tiles = 0;
+    if (use_mfma && part_tokens_override == 0 && part_tiles == 0 && mfma_streamk_plan(p, dtype, &slots, &counters)) {
         p.part_tokens = (int32_t)(max_tiles * 16);
         p.max_parts = 1;
         const int64_t bytes = slots * ((int64_t)p.head_dim + 2) * 4;
         if (bytes >= ((int64_t)1 << 31)) throw PamError("stream-K workspace exceeds 2 GiB");
         if (fixed) {
-            if (bytes > fixed_parts) throw too_big("split-context partials", bytes, fixed_parts);
-            if (counters * 8 > (int64_t)kNoAllocCounterBytes)
-                throw too_big("merge counters", counters * 8, (int64_t)kNoAllocCounterBytes);
             p.part_o = reinterpret_cast<float *>(fixed + kNoAllocZeroBytes + kNoAllocCounterBytes);
             p.seg_count = reinterpret_cast<uint64_t *>(fixed + kNoAllocZeroBytes);
         } else {
@@ -411,7 +468,7 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
             return t >= max_tiles ? (int64_t)0
                                   : p.rows * (int64_t)p.num_heads * ceil_div(max_tiles, t) * (p.head_dim + 2) * 4;
         };
-        while (fixed && bytes_of(tpp) > fixed_parts) tpp *= 2;
+        while (bytes_of(tpp) > (fixed ? fixed_parts : ((int64_t)1 << 31) - 1)) tpp *= 2;
         p.row_blocks = 1;
         p.part_tokens = (int32_t)(std::min(tpp, max_tiles) * 16);
         p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(max_tiles, tpp));
@@ -426,7 +483,7 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
         p.part_ml = p.part_o + (int64_t)p.rows * p.num_heads * p.max_parts * p.head_dim;
         return bytes;
     }
-    p.part_tokens = choose_part_tokens(waves, max_tiles, use_mfma);
+    p.part_tokens = part_tiles > 0 ? (int32_t)(part_tiles * 16) : choose_part_tokens(waves, max_tiles, use_mfma);
     p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(max_tiles, p.part_tokens / 16));
     if (p.max_parts <= 1) return 0;
     // VALU rows of one or two heads per wave split into at most kValuWgMaxParts
@@ -436,7 +493,7 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
         p.valu_wg = 1;
         return 0;
     }
-    const int64_t slots_p = (int64_t)p.rows * p.num_heads * p.max_parts;
+    const int64_t slots_p = (int64_t)p.rows * p.num_heads * layers * p.max_parts;
     const int64_t bytes = slots_p * ((int64_t)p.head_dim + 2) * 4;
     if (bytes >= ((int64_t)1 << 31)) throw PamError("split-context workspace exceeds 2 GiB");
     // The VALU kernel merges its partitions itself (one counter per row and
@@ -576,8 +633,10 @@ void Context::module_load(const char *path) {
     t.prefill[1][0] = get("pam_prefill_f16_d64");
     t.prefill[1][1] = get("pam_prefill_fused_f16_d64");
     t.prefill[1][2] = get("pam_prefill_e4m3_d64");
-    t.mfma_wg[0] = get("pam_decode_wg_f16_d128");
-    t.mfma_wg[1] = get("pam_decode_wg_e4m3_d128");
+    t.mfma_wg[0][0] = get("pam_decode_wg_f16_d128");
+    t.mfma_wg[1][0] = get("pam_decode_wg_e4m3_d128");
+    t.mfma_wg[0][1] = get("pam_decode_layers_wg_f16_d128");
+    t.mfma_wg[1][1] = get("pam_decode_layers_wg_e4m3_d128");
     t.mixed[0] = get("pam_mixed_step_f16_d128");
     t.mixed[1] = get("pam_mixed_step_e4m3_d128");
     static const char *kv_names[3] = {"f32", "f16", "e4m3"};
@@ -595,6 +654,7 @@ void Context::module_load(const char *path) {
             t.decode_rows[k][w] = get(("pam_decode_rows_" + std::string(kv_names[k]) + "_d" + dims[w]).c_str());
     t.reduce[0] = get("pam_reduce_f32");
     t.reduce[1] = get("pam_reduce_f16");
+    t.reduce[2] = get("pam_reduce_layers_f16");
     static const char *piece[3] = {"16", "4", "2"};
     for (int w = 0; w < 3; w++) {
         t.append[w] = get(("pam_append_b" + std::string(piece[w])).c_str());
@@ -760,7 +820,6 @@ Context::DecodePlan Context::plan_decode(const pam_decode_request &r, char *fixe
     if (l.window_size > 0) max_tiles = std::min<int64_t>(max_tiles, l.window_size / 16 + 2);
     const int64_t waves = (int64_t)r.batch_size * (use_mfma ? l.num_kv_heads : l.num_heads / nh);
     d.tmp = plan_split(p, l.data_type, use_mfma, max_tiles, waves, fixed);
-    if (fused > 1 && p.seg_count == nullptr) throw PamError("decode layers cannot be fused");
     d.use_mfma = use_mfma;
     return d;
 }
@@ -1161,10 +1220,14 @@ int64_t Context::plan_prefill_rows(AttnParams &p, int32_t dtype) {
                                              : prefill_rows_part_tokens(p, dtype, cus_);
     const int64_t kv_len = (int64_t)p.q_offset + p.rows;
     const int64_t k_lo = p.window > 0 && kv_len > p.window ? kv_len - p.window : 0;
-    p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(ceil_div(kv_len, 16) - k_lo / 16, p.part_tokens / 16));
-    if (p.max_parts <= 1) return 0;
-    const int64_t slots = (int64_t)p.rows * p.num_heads * p.max_parts;
-    const int64_t bytes = slots * ((int64_t)p.head_dim + 2) * 4;
+    int64_t slots = 0, bytes = 0;
+    for (;; p.part_tokens *= 2) {  // partials under 2 GiB
+        p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(ceil_div(kv_len, 16) - k_lo / 16, p.part_tokens / 16));
+        if (p.max_parts <= 1) return 0;
+        slots = (int64_t)p.rows * p.num_heads * p.max_parts;
+        bytes = slots * ((int64_t)p.head_dim + 2) * 4;
+        if (bytes < ((int64_t)1 << 31)) break;
+    }
     reserve_workspace((size_t)bytes);
     p.part_o = static_cast<float *>(workspace_.ptr);
     p.part_ml = p.part_o + slots * p.head_dim;

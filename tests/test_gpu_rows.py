@@ -202,3 +202,52 @@ def test_decode_rows_code_object_bit_identical(dtype, d, lens):
 def test_backward_rows_parity(dtype, T, H, hkv, d, bs, W):
     import test_gpu_backward
     test_gpu_backward.test_backward_parity(dtype, T, H, hkv, d, bs, W)
+
+
+# MFMA decode as partitions (mfma_part_tiles): one partition, and the shortest and
+# longest partition lengths the rule picks, on both sides of its lines
+@pytest.mark.parametrize("dtype,H,hkv,d,bs,lens,window", [
+    (1, 32, 8, 128, 16, [512, 1, 0, 300], 0),        # 32 tiles: one partition
+    (1, 32, 8, 128, 16, [513, 17], 0),               # 33 tiles: 128-token partitions
+    (1, 8, 1, 128, 16, [8200], 0),                   # 512-token partitions, the last of 8 tokens
+    (1, 32, 8, 64, 8, [2000] + [5] * 20, 0),         # 8-token blocks, most rows in the first partition
+    (1, 64, 8, 256, 16, [256, 2, 40], 0),
+    (1, 64, 8, 256, 16, [257, 100], 0),
+    (2, 32, 8, 128, 16, [1500, 100, 16, 0], 0),
+    (2, 16, 4, 64, 32, [3000, 7], 900),
+    (1, 16, 4, 128, 16, [5000] * 3, 700),
+])
+def test_decode_partitions_parity(dtype, H, hkv, d, bs, lens, window):
+    test_decode_rows_parity(dtype, H, hkv, d, bs, lens, window, 0)
+
+
+@pytest.mark.parametrize("dtype,d,lens", [(1, 128, [700, 0, 40]), (2, 128, [90, 300]), (1, 64, [2000, 1])])
+def test_decode_layers_partitions_bit_identical(dtype, d, lens):
+    """Layers fused over partitions (and their reduce) against single-layer decodes,
+    from the library and (d = 128) from the code object."""
+    import torch
+    H, hkv, bs, n = 32, 8, 16, 3
+    rng = np.random.default_rng(81)
+    q, k, v, bt, lens = make_case(rng, len(lens), H, hkv, d, bs, dtype, lens)
+    ksd = vsd = None
+    if dtype == 2:
+        kd, vd, ksd, vsd, *_ = build_fp8(_engine(), rng, k, v, bt, lens, hkv, d, bs)
+    else:
+        kd, vd = to_dev(k), to_dev(v)
+    qs = [to_dev(rng.standard_normal(q.shape).astype(np.float16)) for _ in range(n)]
+    btd, lnd, lay = to_dev(bt), to_dev(lens), layer(H, hkv, d, bs, dtype)
+    single = []
+    eng = _engine()
+    for x in qs:
+        o = torch.empty(q.shape, dtype=torch.float16, device="cuda")
+        eng.decode(x, kd, vd, btd, lnd, o, len(lens), bt.shape[1], lay, k_scale=ksd, v_scale=vsd)
+        single.append(to_host(o))
+    for module in (False, True) if d == 128 else (False,):
+        eng = _engine()
+        if module:
+            eng.load_module()
+            eng.set_module_strict(True)
+        outs = [torch.empty(q.shape, dtype=torch.float16, device="cuda") for _ in range(n)]
+        eng.decode_layers(qs, kd, vd, btd, lnd, outs, len(lens), bt.shape[1], [lay] * n, k_scale=ksd, v_scale=vsd)
+        for a, b in zip(single, outs):
+            assert np.array_equal(a.view(np.uint16), to_host(b).view(np.uint16))

@@ -346,22 +346,43 @@ __device__ __forceinline__ void valu_body(const AttnParams &p, int lanes_per_row
 // partials' maxima and sums are reduced across lanes (one partition per lane),
 // then lane groups of HD/4 lanes each accumulate a share of the partitions'
 // weighted outputs and the groups are summed with shuffles.
+//
+// What bounds it: latency, of the row's length and of the partials behind it.  The
+// first partials' loads (kReduceAhead a lane: 16 partitions at d = 128) and their
+// maxima are therefore issued before the length is known, within max_parts, and
+// dropped where the row has fewer: 258 small decodes (1-64 rows, 100-4000 tokens)
+// took 4% less on average, with the early window of mfma_item.
+constexpr int kReduceAhead = 8;
 template <typename QT, bool FL = false>
 __device__ __forceinline__ void reduce_body(const AttnParams &p) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = blockIdx.y, h = blockIdx.x * 4 + wave;
     const int G = slot_group<FL>(p), H = G * p.num_kv_heads;  // query-head slots
     if (h >= H) return;
+    const int HD = p.head_dim, most = p.max_parts;
+    const int64_t base = ((int64_t)r * H + h) * most;
+    // lanes per group: HD/4 rounded up to a power of two (<= 64)
+    int lpg = 1;
+    while (lpg * 4 < HD) lpg <<= 1;
+    const int ng = 64 / lpg, g = lane / lpg, d0 = (lane % lpg) * 4;
+    const int na = lpg < kReduceAhead ? lpg : kReduceAhead;  // at most 64 partitions ahead: those of ml0
+    const f32x2 ml0 = *reinterpret_cast<const f32x2 *>(p.part_ml + (base + (lane < most ? lane : most - 1)) * 2);
+    float4 ahead[kReduceAhead];
+#pragma unroll
+    for (int u = 0; u < kReduceAhead; u++)
+        if (u < na && u * ng < most) {
+            const int i = g + u * ng;
+            ahead[u] = *reinterpret_cast<const float4 *>(p.part_o + (base + (i < most ? i : most - 1)) * HD +
+                                                         (d0 < HD ? d0 : 0));
+        }
     const RowCtx c = row_ctx(p, r);
     const PartRange pr = part_range(c, 0, p.part_tokens);
     const int np = pr.nparts;
     if (np <= 1) return;
-    const int HD = p.head_dim;
-    const int64_t base = ((int64_t)r * H + h) * p.max_parts;
     // one pass over (m, l): each lane folds its partitions, then the lanes merge
     float Ml = -INFINITY, dl = 0.0f;
     for (int i = lane; i < np; i += 64) {
-        const float mi = p.part_ml[(base + i) * 2], li = p.part_ml[(base + i) * 2 + 1];
+        const float mi = i < 64 ? ml0[0] : p.part_ml[(base + i) * 2], li = i < 64 ? ml0[1] : p.part_ml[(base + i) * 2 + 1];
         const float Mn = fmaxf(Ml, mi);
         if (Mn != -INFINITY) dl = dl * exp2f(Ml - Mn) + li * exp2f(mi - Mn);
         Ml = Mn;
@@ -369,14 +390,20 @@ __device__ __forceinline__ void reduce_body(const AttnParams &p) {
     const float M = wave_max_xor(Ml, 1, 64);
     float den = Ml == -INFINITY ? 0.0f : dl * exp2f(Ml - M);
     den = wave_sum_xor(den, 1, 64);
-    // lanes per group: HD/4 rounded up to a power of two (<= 64)
-    int lpg = 1;
-    while (lpg * 4 < HD) lpg <<= 1;
-    const int ng = 64 / lpg, g = lane / lpg, d0 = (lane % lpg) * 4;
     float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kReduceAhead; u++) {
+        if (u >= na || u * ng >= np) break;
+        const int i = g + u * ng;
+        const float w = exp2f(__shfl(ml0[0], i & 63, 64) - M);
+        if (i < np) {
+            a[0] += w * ahead[u].x, a[1] += w * ahead[u].y;
+            a[2] += w * ahead[u].z, a[3] += w * ahead[u].w;
+        }
+    }
     if (d0 < HD) {
 #pragma unroll 4
-        for (int i = g; i < np; i += ng) {
+        for (int i = g + na * ng; i < np; i += ng) {
             const float w = exp2f(p.part_ml[(base + i) * 2] - M);
             float v[4];
             load4<float>(p.part_o + (base + i) * HD + d0, v);

@@ -3,11 +3,12 @@
 // matrix kernels do not take (other head sizes, groups that are no power of two).
 //
 // The semantics and the split of the work are backward.hip's, without atomics:
-//   * bwd_dq_rows: a workgroup owns 16 query rows (token, head) of one kv head;
-//     its waves take the 16-key tiles in turn, once for D_i = sum_j P_ij
-//     dP_ij and once for dQ^T += K^T dS^T, and sum in LDS;
-//   * bwd_dkv_rows: a workgroup owns 16 keys of one kv head and one share of the
-//     group's query rows; its waves take the 16-row tiles in turn for
+//   * bwd_d_rows: a workgroup owns one or two blocks of 16 query rows (token, head)
+//     of one kv head; its waves take the 16-key tiles in turn for
+//     D_i = sum_j P_ij dP_ij and sum in LDS;
+//   * bwd_grads_rows: workgroups of such row blocks, whose waves take the key tiles
+//     in turn for dQ^T += K^T dS^T, and workgroups of key blocks, each with one
+//     share of the group's query rows, whose waves take the 16-row tiles in turn for
 //     dV^T += dO^T P and dK^T += Q^T dS.  Shares of one key block go through f32
 //     partials that bwd_dkv_sum adds to the gradient pools in order.
 // The arrangement is rows_body.h's: S and dP on v_mfma_f32_16x16x4_f32 (f16:
@@ -18,13 +19,15 @@
 // and by dims (VW dims of one row) for the gradients.
 //
 // What bounds it: the f32 matrix rate (nine products over the (row, key) pairs
-// where five are needed: two kernels recompute S and dP, and D needs its own
-// pass); a short sequence, its few workgroups and the latency of its tiles' loads.
-// Measured on gfx950 against the VALU kernels, which served these shapes before (µs
-// per call): f32 8/2 d = 64, 600 tokens 2140 -> 98 (dQ 45, dK / dV 43, sum 5); f32
-// 16/4 d = 64, 1000 tokens 7160 -> 243; f16 8/8 d = 64, 1000 tokens 3700 -> 76; f16
-// 32/8 d = 64, 2000 tokens 50300 -> 865 (95 TFLOP/s of the five products).  One
-// block of rows or keys a wave in place of two: 322, 106 and 1124 for the last three.
+// where five are needed: S and dP are formed for D, for dQ and for dK / dV); a
+// short sequence, its few workgroups and the latency of its tiles' loads.  Measured
+// on gfx950 against the VALU kernels, which served these shapes before (µs per
+// call): f32 8/2 d = 64, 600 tokens 2500 -> 78 (D 21, gradients 52, sum 5); f32 16/4
+// d = 64, 1000 tokens 7160 -> 247; f16 8/8 d = 64, 1000 tokens 3700 -> 77; f16 32/8
+// d = 64, 2000 tokens 50300 -> 847 (97 TFLOP/s of the five products).  One block of
+// rows or keys a wave in place of two: 322, 106 and 1124 for the last three; D alone
+// with one: 259, 83 and 940.  dQ (with D) and dK / dV in launches of their own, where
+// each leaves CUs idle: 94, 246, 76 and 858; 12/4 d = 96, 200 tokens 50 against 40.
 #include "rows_body.h"
 
 namespace pam {
@@ -148,103 +151,158 @@ __device__ __forceinline__ void lds_sum(const float *lds, int rn, int e0, float 
     }
 }
 
-template <typename T, class S>
-__global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_dq_rows(BackwardParams p) {
-    constexpr int B = S::BQ, W = S::W, LS = S::LS;
-    __shared__ __attribute__((aligned(16))) float lds[W * 16 * LS];
+// row of q and d_out of the group's row rho (-1: past the end)
+__device__ __forceinline__ int query_row(const BackwardParams &p, int kvh, int rho) {
+    const int H = p.num_heads, G = H / p.num_kv_heads;
+    return rho < p.seq_len * G ? rho / G * H + kvh * G + rho % G : -1;
+}
+
+// The row terms, D among them.  grid: kv head + Hkv * (16 B rows).
+template <typename T, class S, int B>
+__global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_d_rows(BackwardParams p) {
+    constexpr int W = S::W;
     __shared__ float d_lds[W][16 * B];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
-    const int H = p.num_heads, Hkv = p.num_kv_heads, G = H / Hkv, d = p.head_dim;
-    const int kvh = blockIdx.x % Hkv, row0 = (int)(blockIdx.x / Hkv) * 16 * B, rows = p.seq_len * G;
+    const int Hkv = p.num_kv_heads, d = p.head_dim;
+    const int kvh = blockIdx.x % Hkv, row0 = (int)(blockIdx.x / Hkv) * 16 * B, rows = p.seq_len * (p.num_heads / Hkv);
     const char *zero = static_cast<const char *>(p.zero_page);
     const int64_t q_bytes = (int64_t)d * (int)sizeof(T), kv_bytes = Hkv * q_bytes;
     const char *kbase = static_cast<const char *>(p.k_pool) + kvh * q_bytes, *vbase = static_cast<const char *>(p.v_pool) + kvh * q_bytes;
     RowOp<T, S> q[B], go[B];
     float m[B], inv_l[B], D[B];
-    f32x4 dq[B][2 * S::NT];
 #pragma unroll
     for (int b = 0; b < B; b++) {
-        const int rho = row0 + 16 * b + n;
-        const int so = rho < rows ? rho / G * H + kvh * G + rho % G : -1;
+        const int so = query_row(p, kvh, row0 + 16 * b + n);
         q[b].load(at_row(static_cast<const char *>(p.q), so, q_bytes, zero), g, d, zero);
         go[b].load(at_row(static_cast<const char *>(p.d_out), so, q_bytes, zero), g, d, zero);
         m[b] = p.m[so < 0 ? 0 : so];
         inv_l[b] = 1.0f / p.l[so < 0 ? 0 : so];
         D[b] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 2 * S::NT; i++) dq[b][i] = (f32x4)0.0f;
     }
     const KeySlots keys(p);
-    const int t0 = p.window_start / 16, t1 = (p.seq_len + 15) / 16, first = t0 + wave;
+    const int t1 = (p.seq_len + 15) / 16, first = p.window_start / 16 + wave;
     auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : -1; };
+    RowOp<T, S> k, v;
+    int slot = slot_of(first), ahead = slot_of(first + W);
+    if (first < t1) {
+        k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
+        v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
+    }
+    for (int t = first; t < t1; t += W) {
+        f32x4 s[B], dp[B];
 #pragma unroll
-    for (int pass = 0; pass < 2; pass++) {
-        RowOp<T, S> k, v;
-        int slot = slot_of(first), ahead = slot_of(first + W);
-        if (first < t1) {
+        for (int b = 0; b < B; b++) s[b] = RowOp<T, S>::dot(k, q[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool more = t + W < t1;
+        slot = ahead;
+        if (more) {
+            ahead = slot_of(t + 2 * W);
             k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
-            v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
         }
-        for (int t = first; t < t1; t += W) {
-            DimOp<T, S> kd[4];
-            if (pass) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    kd[r].load(at_row(kbase, __shfl(slot, 4 * g + r, 64), kv_bytes, zero), n, d, zero);
-            }
-            f32x4 s[B], dp[B];
+        for (int b = 0; b < B; b++) dp[b] = RowOp<T, S>::dot(v, go[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool edge = 16 * t < p.window_start || 16 * t + 16 > p.seq_len;
 #pragma unroll
-            for (int b = 0; b < B; b++) s[b] = RowOp<T, S>::dot(k, q[b]);
-            __builtin_amdgcn_sched_barrier(0);
-            const bool more = t + W < t1;
-            slot = ahead;
-            if (more) {
-                ahead = slot_of(t + 2 * W);
-                k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int b = 0; b < B; b++) dp[b] = RowOp<T, S>::dot(v, go[b]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (more) v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
-            __builtin_amdgcn_sched_barrier(0);
-            const bool edge = 16 * t < p.window_start || 16 * t + 16 > p.seq_len;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int j = 16 * t + 4 * g + r;
-                float dS[B];
-#pragma unroll
-                for (int b = 0; b < B; b++) {
-                    float P = prob(s[b][r], p.scale, m[b], inv_l[b]);
-                    if (edge) P = j >= p.window_start && j < p.seq_len ? P : 0.0f;
-                    if (pass)
-                        dS[b] = P * (dp[b][r] - D[b]);
-                    else
-                        D[b] = fmaf(P, dp[b][r], D[b]);
-                }
-                if (pass) kd[r].add(dS, dq);
-            }
-        }
-        if (!pass) {
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * t + 4 * g + r;
 #pragma unroll
             for (int b = 0; b < B; b++) {
-                D[b] += shfl_xor(D[b], 16);
-                D[b] += shfl_xor(D[b], 32);
-                if (g == 0) d_lds[wave][16 * b + n] = D[b];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int b = 0; b < B; b++) {
-                D[b] = 0.0f;
-#pragma unroll
-                for (int w = 0; w < W; w++) D[b] += d_lds[w][16 * b + n];
+                float P = prob(s[b][r], p.scale, m[b], inv_l[b]);
+                if (edge) P = j >= p.window_start && j < p.seq_len ? P : 0.0f;
+                D[b] = fmaf(P, dp[b][r], D[b]);
             }
         }
     }
 #pragma unroll
     for (int b = 0; b < B; b++) {
+        D[b] += shfl_xor(D[b], 16);
+        D[b] += shfl_xor(D[b], 32);
+        if (g == 0) d_lds[wave][16 * b + n] = D[b];
+    }
+    __syncthreads();
+    if (wave != 0 || g != 0) return;
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        D[b] = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; w++) D[b] += d_lds[w][16 * b + n];
+        const int rho = row0 + 16 * b + n;
+        if (rho < rows) row_terms(p, kvh)[rho] = make_float4(m[b], inv_l[b], D[b], 0.0f);
+    }
+}
+
+// dQ of workgroup id: kv head + Hkv * (16 BQ rows)
+template <typename T, class S>
+__device__ __forceinline__ void dq_rows_body(const BackwardParams &p, int id, float *lds) {
+    constexpr int B = S::BQ, W = S::W, LS = S::LS;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int H = p.num_heads, Hkv = p.num_kv_heads, G = H / Hkv, d = p.head_dim;
+    const int kvh = id % Hkv, row0 = id / Hkv * 16 * B, rows = p.seq_len * G;
+    const char *zero = static_cast<const char *>(p.zero_page);
+    const int64_t q_bytes = (int64_t)d * (int)sizeof(T), kv_bytes = Hkv * q_bytes;
+    const char *kbase = static_cast<const char *>(p.k_pool) + kvh * q_bytes, *vbase = static_cast<const char *>(p.v_pool) + kvh * q_bytes;
+    RowOp<T, S> q[B], go[B];
+    float4 rt[B];
+    f32x4 dq[B][2 * S::NT];
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        const int rho = row0 + 16 * b + n, so = query_row(p, kvh, rho);
+        q[b].load(at_row(static_cast<const char *>(p.q), so, q_bytes, zero), g, d, zero);
+        go[b].load(at_row(static_cast<const char *>(p.d_out), so, q_bytes, zero), g, d, zero);
+        rt[b] = row_terms(p, kvh)[rho < rows ? rho : rows - 1];
+#pragma unroll
+        for (int i = 0; i < 2 * S::NT; i++) dq[b][i] = (f32x4)0.0f;
+    }
+    const KeySlots keys(p);
+    const int t1 = (p.seq_len + 15) / 16, first = p.window_start / 16 + wave;
+    auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : -1; };
+    RowOp<T, S> k, v;
+    int slot = slot_of(first), ahead = slot_of(first + W);
+    if (first < t1) {
+        k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
+        v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
+    }
+    for (int t = first; t < t1; t += W) {
+        DimOp<T, S> kd[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) kd[r].load(at_row(kbase, __shfl(slot, 4 * g + r, 64), kv_bytes, zero), n, d, zero);
+        f32x4 s[B], dp[B];
+#pragma unroll
+        for (int b = 0; b < B; b++) s[b] = RowOp<T, S>::dot(k, q[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool more = t + W < t1;
+        slot = ahead;
+        if (more) {
+            ahead = slot_of(t + 2 * W);
+            k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < B; b++) dp[b] = RowOp<T, S>::dot(v, go[b]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool edge = 16 * t < p.window_start || 16 * t + 16 > p.seq_len;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * t + 4 * g + r;
+            float dS[B];
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                float P = prob(s[b][r], p.scale, rt[b].x, rt[b].y);
+                if (edge) P = j >= p.window_start && j < p.seq_len ? P : 0.0f;
+                dS[b] = P * (dp[b][r] - rt[b].z);
+            }
+            kd[r].add(dS, dq);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < B; b++) {
         const int rb = row0 + 16 * b;
-        if (wave == 0 && g == 0 && rb + n < rows) row_terms(p, kvh)[rb + n] = make_float4(m[b], inv_l[b], D[b], 0.0f);
         if (b) __syncthreads();
         DimOp<T, S>::put(dq[b], g, lds + (wave * 16 + n) * LS);
         __syncthreads();
@@ -272,13 +330,13 @@ __device__ __forceinline__ void pool_add(void *pool, const BackwardParams &p, co
     store4<T>(row, x);
 }
 
+// dK / dV of workgroup id: kv head + Hkv * (16 BK keys), and a share of the rows
 template <typename T, class S>
-__global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_dkv_rows(BackwardParams p) {
+__device__ __forceinline__ void dkv_rows_body(const BackwardParams &p, int id, int share, float *lds) {
     constexpr int B = S::BK, W = S::W, LS = S::LS;
-    __shared__ __attribute__((aligned(16))) float lds[W * 16 * LS];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int H = p.num_heads, Hkv = p.num_kv_heads, G = H / Hkv, d = p.head_dim;
-    const int kvh = blockIdx.x % Hkv, key0 = p.window_start + (int)(blockIdx.x / Hkv) * 16 * B, rows = p.seq_len * G;
+    const int kvh = id % Hkv, key0 = p.window_start + id / Hkv * 16 * B, rows = p.seq_len * G;
     const char *zero = static_cast<const char *>(p.zero_page), *Q = static_cast<const char *>(p.q),
                *dO = static_cast<const char *>(p.d_out);
     const int64_t q_bytes = (int64_t)d * (int)sizeof(T), kv_bytes = Hkv * q_bytes;
@@ -295,7 +353,7 @@ __global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_dkv_rows(
     }
     const float4 *terms = row_terms(p, kvh);
     const int tiles = (rows + 15) / 16, per = (tiles + p.shares - 1) / p.shares;
-    const int t0 = (int)blockIdx.y * per, t1 = t0 + per < tiles ? t0 + per : tiles;
+    const int t0 = share * per, t1 = t0 + per < tiles ? t0 + per : tiles;
     // row of q and d_out of the group's row rho (-1: past the end)
     const int gs = block_shift(G);
     auto row_of = [&](int rho) {
@@ -374,12 +432,24 @@ __global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_dkv_rows(
                     for (int e = 0; e < 4; e++) a[e] *= p.scale;
                 if (p.shares > 1) {
                     const int64_t nk = p.seq_len - p.window_start, row = (int64_t)(j - p.window_start) * Hkv + kvh;
-                    store4<float>(p.partial + ((int64_t)(2 * blockIdx.y + which) * nk * Hkv + row) * d + e0, a);
+                    store4<float>(p.partial + ((int64_t)(2 * share + which) * nk * Hkv + row) * d + e0, a);
                 } else {
                     pool_add<T>(which ? p.d_v_pool : p.d_k_pool, p, keys, j, kvh, e0, a);
                 }
             }
         }
+}
+
+// Both sides of the gradients in one launch, so that neither waits for the other's
+// last workgroups: the first n_dq workgroups take dQ, the others dK / dV.
+template <typename T, class S>
+__global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_grads_rows(BackwardParams p, int n_dq) {
+    __shared__ __attribute__((aligned(16))) float lds[S::W * 16 * S::LS];
+    const int id = blockIdx.x;
+    if (id < n_dq)
+        dq_rows_body<T, S>(p, id, lds);
+    else
+        dkv_rows_body<T, S>(p, (id - n_dq) / p.shares, (id - n_dq) % p.shares, lds);
 }
 
 // the shares' partials, summed in order, into the gradient pools
@@ -455,14 +525,12 @@ static hipError_t launch_type(const BackwardParams &p, hipStream_t stream) {
         const int64_t rows = (int64_t)p.seq_len * (p.num_heads / p.num_kv_heads), keys = p.seq_len - p.window_start;
         const int64_t rspan = 16 * S::BQ, kspan = 16 * S::BK;
         const dim3 block(64 * S::W);
-        hipLaunchKernelGGL((bwd_dq_rows<T, S>), dim3((unsigned)((rows + rspan - 1) / rspan * p.num_kv_heads)), block, 0,
-                           stream, p);
-        if (keys > 0) {
-            hipLaunchKernelGGL((bwd_dkv_rows<T, S>),
-                               dim3((unsigned)((keys + kspan - 1) / kspan * p.num_kv_heads), (unsigned)p.shares), block, 0,
-                               stream, p);
-            if (p.shares > 1) return launch_backward_sum(p, sizeof(T) == 4 ? kF32 : kF16, stream);
-        }
+        const int64_t n_dq = (rows + rspan - 1) / rspan * p.num_kv_heads;
+        const int64_t n_dkv = (keys + kspan - 1) / kspan * p.num_kv_heads * p.shares;
+        if (n_dq + n_dkv >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((bwd_d_rows<T, S, S::BQ>), dim3((unsigned)n_dq), block, 0, stream, p);
+        hipLaunchKernelGGL((bwd_grads_rows<T, S>), dim3((unsigned)(n_dq + n_dkv)), block, 0, stream, p, (int)n_dq);
+        if (keys > 0 && p.shares > 1) return launch_backward_sum(p, sizeof(T) == 4 ? kF32 : kF16, stream);
         return hipGetLastError();
     });
 }

@@ -31,6 +31,11 @@ constexpr int kMaxFusedLayers = 4;
 // most partitions of the VALU kernel's workgroup form (one wave each)
 constexpr int kValuWgMaxParts = 16;
 
+// most rows or partitions of the row-block kernels and their reduce, which lie in
+// the y and z dimensions of a grid; more decode rows keep the VALU kernel, more
+// prefill rows one partition
+constexpr int64_t kMaxGridYZ = 65535;
+
 struct AttnParams {
     const void *q;             // [rows][H][d] (f32 for f32 caches, f16 otherwise)
     void *out;                 // [rows][H][d] same type as q
@@ -144,7 +149,8 @@ hipError_t streamk_occupancy(int32_t dtype, bool fused_layers, int *per_cu);
 
 // Paged attention over rows (decode / prefill-as-rows / ragged).  Chooses the
 // MFMA kernel for 4 <= H/Hkv <= 16 with f16/fp8 KV and d in {64,128,256},
-// otherwise the VALU kernel.  Launches the split-context reduce when max_parts > 1.
+// otherwise the row-block kernels (row_blocks) or the VALU kernel.  Launches the
+// split-context reduce when max_parts > 1.
 hipError_t launch_attention(const AttnParams &p, int32_t dtype, bool use_mfma, hipStream_t stream,
                             hipEvent_t after_main = nullptr, const KernelTable *kt = nullptr);
 bool mfma_supported(int32_t dtype, int32_t head_dim, int32_t group, int32_t block_size);

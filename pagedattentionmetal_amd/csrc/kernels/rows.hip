@@ -97,7 +97,7 @@ static hipError_t launch_rows(const AttnParams &p, hipStream_t stream, const Ker
     hipError_t me;
     if (p.mode == kRowPrefill) {
         const int64_t R = block_rows(p.head_dim, kvi == 0 ? kF32 : kF16), nblocks = ((int64_t)p.rows * G + R - 1) / R;
-        if (nblocks * p.num_kv_heads >= ((int64_t)1 << 31) || p.rows * G >= ((int64_t)1 << 31) - 32 || parts > 65535)
+        if (nblocks * p.num_kv_heads >= ((int64_t)1 << 31) || p.rows * G >= ((int64_t)1 << 31) - 32 || parts > kMaxGridYZ)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned)(nblocks * p.num_kv_heads), (unsigned)parts);
         if (via_module(kt, kt ? kt->prefill_rows[kvi][dim_slot(p.head_dim)] : nullptr, &me, grid, block, stream, p)) return me;
@@ -105,7 +105,7 @@ static hipError_t launch_rows(const AttnParams &p, hipStream_t stream, const Ker
         return hipGetLastError();
     }
     const int64_t slots = p.num_kv_heads * ((G + 15) / 16);
-    if (p.rows > 65535 || parts > 65535) return hipErrorInvalidValue;
+    if (p.rows > kMaxGridYZ || parts > kMaxGridYZ) return hipErrorInvalidValue;
     const dim3 grid((unsigned)slots, (unsigned)p.rows, (unsigned)parts);
     if (via_module(kt, kt ? kt->decode_rows[kvi][dim_slot(p.head_dim)] : nullptr, &me, grid, block, stream, p)) return me;
     PAM_ROWS_SWITCH(decode_rows_kernel)

@@ -24,9 +24,9 @@
 // is 2048 matrix cycles for 16 KB in f32, 1150 for 8 KB in f16), and, for e4m3,
 // the f32 matrix time of O^T.  Measured on gfx950 against the VALU rows that
 // served these calls before (µs per call): f32 8/8 d = 128, 777 tokens after 391
-// 784 -> 61 (40 TFLOP/s); f32 32/8 d = 128, 2048 tokens 379 (91 TFLOP/s); f16
+// 784 -> 54 (45 TFLOP/s); f32 32/8 d = 128, 2048 tokens 379 (91 TFLOP/s); f16
 // 32/8 d = 96, 2048 tokens 166 (155 TFLOP/s); f16 16/16 d = 64 decode of 24 rows
-// of up to 3000 tokens 162 -> 49 (3.3 TB/s); f32 8/8 d = 128 64 rows of up to
+// of up to 3000 tokens 162 -> 48 (3.4 TB/s); f32 8/8 d = 128 64 rows of up to
 // 2000 128 -> 117 (4.9 TB/s); f32 32/8 one row of 5598 337 -> 12; e4m3 12/4
 // d = 128 205 rows of up to 4000 2620 -> 172.
 #pragma once
@@ -188,19 +188,22 @@ struct RowTiles {
         for (int t = t0; t < t1; t += step) {
             const int kb = keys.key0 + 16 * t;
             const bool more = t + step < t1;
-            f32x4 s[RB], s2[RB];  // f32: two chains of sums, which halves their rounding
+            // f32: the scores in several chains of sums, added pairwise, for less
+            // rounding than one long chain; as many as cost no resident wave
+            constexpr int CH = F32 ? (RB > 1 ? 2 : (NT >= 4 ? 8 : 4)) : 1;
+            f32x4 s[RB], sc[RB][CH];
 #pragma unroll
-            for (int b = 0; b < RB; b++) s[b] = s2[b] = (f32x4)0.0f;
+            for (int b = 0; b < RB; b++)
+#pragma unroll
+                for (int i = 0; i < CH; i++) sc[b][i] = (f32x4)0.0f;
 #pragma unroll
             for (int c = 0; c < KC; c++) {
                 if constexpr (F32) {
 #pragma unroll
-                    for (int e = 0; e < 4; e += 2)
+                    for (int e = 0; e < 4; e++)
 #pragma unroll
-                        for (int b = 0; b < RB; b++) {
-                            s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[b][c][e], s[b], 0, 0, 0);
-                            s2[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e + 1], q[b][c][e + 1], s2[b], 0, 0, 0);
-                        }
+                        for (int b = 0; b < RB; b++)
+                            sc[b][(4 * c + e) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[b][c][e], sc[b][(4 * c + e) % CH], 0, 0, 0);
                 } else {
                     f16x8 a;
                     if constexpr (sizeof(KV) == 1)
@@ -209,7 +212,7 @@ struct RowTiles {
                         a = k[c];
 #pragma unroll
                     for (int b = 0; b < RB; b++)
-                        s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[b][c], s[b], 0, 0, 0);
+                        sc[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[b][c], sc[b][0], 0, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -220,9 +223,14 @@ struct RowTiles {
                 issue_k(p, row_n, blk_n);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (F32)
 #pragma unroll
-                for (int b = 0; b < RB; b++) s[b] += s2[b];
+            for (int b = 0; b < RB; b++) {
+#pragma unroll
+                for (int h = CH / 2; h > 0; h /= 2)
+#pragma unroll
+                    for (int i = 0; i < h; i++) sc[b][i] += sc[b][i + h];
+                s[b] = sc[b][0];
+            }
             // Online softmax.  The reference max of a row moves only when a score
             // passes it by 8, a factor of 2^8 (or the row has none yet): the probabilities
             // are f32, so their scale is free, and most tiles need no reduction across
@@ -265,6 +273,15 @@ struct RowTiles {
                     l[b] += s[b][r];
                 }
             }
+            // f32, one block: a tile's O^T is summed by itself and then added, which
+            // shortens the chains of sums.  Error of a decode against 64 bits, VALU rows /
+            // one chain of outputs and two of scores / this: 32/8 d = 64, 64 rows of up to
+            // 500 tokens 1.24e-7 / 1.66e-7 / 1.29e-7; 8/8 d = 128, 16 rows of up to 600
+            // 1.60e-7 / 1.71e-7 / 1.30e-7; 32/8 d = 128, 4000 tokens 3.1e-7 / 1.8e-7 /
+            // 1.6e-7; up to 100 tokens 1.03e-7 / 1.3e-7 / 1.1e-7 (an f32 ulp is 1.2e-7);
+            // the times are the same.
+            constexpr bool TS = F32 && RB == 1 && NT <= 4;
+            f32x4 ot[TS ? 2 * NT : 1];
             // O^T.  In an edge tile a V element of a key that some row must not see
             // enters only if it is finite (0 * Inf would reach the rows that mask
             // it); add_odd gives the others to the rows that do see the key.
@@ -286,9 +303,14 @@ struct RowTiles {
 #pragma unroll
                 for (int i = 0; i < 2 * NT; i++)
 #pragma unroll
-                    for (int b = 0; b < RB; b++)
-                        o[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[b][r], o[b][i], 0, 0, 0);
+                    for (int b = 0; b < RB; b++) {
+                        f32x4 &dst = TS ? ot[i] : o[b][i];
+                        dst = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[b][r], TS && r == 0 ? (f32x4)0.0f : dst, 0, 0, 0);
+                    }
             }
+            if constexpr (TS)
+#pragma unroll
+                for (int i = 0; i < 2 * NT; i++) o[0][i] += ot[i];
             __builtin_amdgcn_sched_barrier(0);
             if (more) issue_v(p, row_n, blk_n);
         }

@@ -448,7 +448,7 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
         return bytes;
     }
     if (!use_mfma && p.mode != kRowPrefill && decode_kernel_choice != 1 && rows_supported(p, dtype) &&
-        !valu_rows_win(p, dtype, max_tiles)) {
+        p.rows <= kMaxGridYZ && !valu_rows_win(p, dtype, max_tiles)) {
         // Row-block kernel: one workgroup per (row, slot of up to 16 heads,
         // partition).  A row is cut until there are about 8 workgroups per CU, to
         // no less than 256 tokens (a partition's start and the reduce cost more
@@ -468,7 +468,8 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
             return t >= max_tiles ? (int64_t)0
                                   : p.rows * (int64_t)p.num_heads * ceil_div(max_tiles, t) * (p.head_dim + 2) * 4;
         };
-        while (bytes_of(tpp) > (fixed ? fixed_parts : ((int64_t)1 << 31) - 1)) tpp *= 2;
+        while (bytes_of(tpp) > (fixed ? fixed_parts : ((int64_t)1 << 31) - 1) || ceil_div(max_tiles, tpp) > kMaxGridYZ)
+            tpp *= 2;
         p.row_blocks = 1;
         p.part_tokens = (int32_t)(std::min(tpp, max_tiles) * 16);
         p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(max_tiles, tpp));
@@ -1221,12 +1222,12 @@ int64_t Context::plan_prefill_rows(AttnParams &p, int32_t dtype) {
     const int64_t kv_len = (int64_t)p.q_offset + p.rows;
     const int64_t k_lo = p.window > 0 && kv_len > p.window ? kv_len - p.window : 0;
     int64_t slots = 0, bytes = 0;
-    for (;; p.part_tokens *= 2) {  // partials under 2 GiB
+    for (;; p.part_tokens *= 2) {  // partials under 2 GiB, and grids that the kernels and the reduce take
         p.max_parts = (int32_t)std::max<int64_t>(1, ceil_div(ceil_div(kv_len, 16) - k_lo / 16, p.part_tokens / 16));
         if (p.max_parts <= 1) return 0;
         slots = (int64_t)p.rows * p.num_heads * p.max_parts;
         bytes = slots * ((int64_t)p.head_dim + 2) * 4;
-        if (bytes < ((int64_t)1 << 31)) break;
+        if (bytes < ((int64_t)1 << 31) && p.rows <= kMaxGridYZ && p.max_parts <= kMaxGridYZ) break;
     }
     reserve_workspace((size_t)bytes);
     p.part_o = static_cast<float *>(workspace_.ptr);

@@ -248,7 +248,8 @@ class Context {
     hipStream_t own_stream_ = nullptr, ext_stream_ = nullptr;
     bool use_ext_stream_ = false;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr, evmid_ = nullptr, handoff_ = nullptr;
-    // pinned staging ring: kStageSegs segments, each with the event of its last copy
+    // pinned staging ring: kStageSegs segments, each with an event recorded when the
+    // ring leaves it
     static constexpr int kStageSegs = 4;
     hipEvent_t seg_event_[kStageSegs] = {};
     bool seg_used_[kStageSegs] = {};

@@ -109,6 +109,7 @@ def test_rows_code_object_bit_identical(dtype, d):
     (0, 20, 1, 36, 16, [100, 17], 0, 0),                # 20 heads a kv head: two slots, the second of 4
     (0, 4, 4, 256, 8, [1500, 0, 300], 0, 0),
     (0, 2, 2, 4, 1, [3, 40], 0, 0),
+    (0, 4, 2, 16, 16, [3, 17] * 33000, 0, 0),           # more rows than a grid's z takes: the VALU kernel
     (0, 4, 4, 16, 16, [2100, 130], 0, 16),              # 132 partitions: more than the reduce loads ahead
     (1, 16, 16, 64, 16, [3000, 100, 17, 0], 0, 0),
     (1, 8, 4, 128, 16, [2000, 500], 333, 0),

@@ -348,12 +348,12 @@ static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles)
 // table's length (with rows of a byte a dim or two; a wider row is a workgroup's work
 // but no more of its latency).  Measured on gfx950 (µs per call, stream-K /
 // partitions, rows of L / 8 to L tokens, 32/8 heads): f16 d = 128: 1 row L = 2000 18.1
-// / 11.8, 8 rows L = 500 24.2 / 11.3, L = 2000 22.9 / 17.5, 32 rows L = 200 29.3 / 9.3,
-// L = 1000 28.0 / 20.1, 64 rows L = 500 30.7 / 21.9, L = 1000 33.6 / 38.0, 128 rows L =
-// 200 34.1 / 23.6, L = 500 37.6 / 39.6, 16 rows L = 4000 34.2 / 39.0; e4m3 d = 128: 32
-// rows L = 1000 26.0 / 17.4, L = 4000 37.8 / 45.8, 128 rows L = 500 33.2 / 25.2, L =
-// 1000 40.1 / 41.4; f16 d = 64: 32 rows L = 1000 21.3 / 12.6; d = 256 (64/8): 32 rows
-// L = 1000 47.5 / 34.8, 128 rows L = 500 77.5 / 75.1, 256 rows L = 200 74.1 / 93.8.
+// / 10.4, 8 rows L = 500 24.2 / 10.3, L = 2000 22.9 / 15.8, 32 rows L = 200 29.3 / 8.4,
+// L = 1000 28.0 / 18.2, 64 rows L = 500 30.7 / 20.5, L = 1000 33.6 / 38.0, 128 rows L =
+// 200 34.1 / 21.9, L = 500 37.6 / 39.6, 16 rows L = 4000 34.2 / 39.0; e4m3 d = 128: 32
+// rows L = 1000 26.0 / 16.7, L = 4000 37.8 / 45.8, 128 rows L = 500 33.2 / 24.7, L =
+// 1000 40.1 / 41.4; f16 d = 64: 32 rows L = 1000 21.3 / 11.4; d = 256 (64/8): 32 rows
+// L = 1000 47.5 / 33.0, 128 rows L = 500 77.5 / 75.1, 256 rows L = 200 74.1 / 93.8.
 static int64_t mfma_part_tiles(int64_t pairs, int64_t max_tiles, int32_t head_dim, int32_t dtype, int32_t cus) {
     if (max_tiles <= 0) return 0;
     const int64_t row_bytes = std::min<int64_t>(2 * (int64_t)head_dim * elem_bytes(dtype), 512);

@@ -189,8 +189,8 @@ struct RowTiles {
             const int kb = keys.key0 + 16 * t;
             const bool more = t + step < t1;
             // f32: the scores in several chains of sums, added pairwise, for less
-            // rounding than one long chain; as many as cost no resident wave
-            constexpr int CH = F32 ? (RB > 1 ? 2 : (NT >= 4 ? 8 : 4)) : 1;
+            // rounding than one long chain; as many as the registers hold
+            constexpr int CH = F32 ? (RB > 1 ? (NT <= 2 ? 4 : 2) : (NT >= 4 ? 8 : 4)) : 1;
             f32x4 s[RB], sc[RB][CH];
 #pragma unroll
             for (int b = 0; b < RB; b++)
@@ -273,15 +273,18 @@ struct RowTiles {
                     l[b] += s[b][r];
                 }
             }
-            // f32, one block: a tile's O^T is summed by itself and then added, which
-            // shortens the chains of sums.  Error of a decode against 64 bits, VALU rows /
-            // one chain of outputs and two of scores / this: 32/8 d = 64, 64 rows of up to
-            // 500 tokens 1.24e-7 / 1.66e-7 / 1.29e-7; 8/8 d = 128, 16 rows of up to 600
-            // 1.60e-7 / 1.71e-7 / 1.30e-7; 32/8 d = 128, 4000 tokens 3.1e-7 / 1.8e-7 /
-            // 1.6e-7; up to 100 tokens 1.03e-7 / 1.3e-7 / 1.1e-7 (an f32 ulp is 1.2e-7);
-            // the times are the same.
-            constexpr bool TS = F32 && RB == 1 && NT <= 4;
-            f32x4 ot[TS ? 2 * NT : 1];
+            // f32, where the registers hold it: a tile's O^T is summed by itself and then
+            // added, which shortens the chains of sums.  Error against 64 bits, VALU rows
+            // / one chain of outputs and two of scores / this: decode 32/8 d = 64, 64
+            // rows of up to 500 tokens 1.24e-7 / 1.66e-7 / 1.30e-7; 8/8 d = 128, 16 rows
+            // of up to 600 1.60e-7 / 1.71e-7 / 1.30e-7; 32/8 d = 128, 4000 tokens 3.1e-7 /
+            // 1.8e-7 / 1.6e-7; up to 100 tokens 1.03e-7 / 1.3e-7 / 1.1e-7 (an f32 ulp is
+            // 1.2e-7); prefill d = 64 32/8, 874 tokens 1.14e-7 / 1.37e-7 / 1.05e-7, 8/8,
+            // 777 after 391 1.86e-7 / 2.14e-7 / 1.49e-7.  Times (µs per call, without /
+            // with): those decodes the same; the prefills 51 / 58 (554 on the VALU rows)
+            // and 33 / 33, 8/2 2048 tokens 84 / 82.
+            constexpr bool TS = F32 && NT <= (RB == 1 ? 4 : 2);
+            f32x4 ot[RB][TS ? 2 * NT : 1];
             // O^T.  In an edge tile a V element of a key that some row must not see
             // enters only if it is finite (0 * Inf would reach the rows that mask
             // it); add_odd gives the others to the rows that do see the key.
@@ -304,13 +307,15 @@ struct RowTiles {
                 for (int i = 0; i < 2 * NT; i++)
 #pragma unroll
                     for (int b = 0; b < RB; b++) {
-                        f32x4 &dst = TS ? ot[i] : o[b][i];
+                        f32x4 &dst = TS ? ot[b][i] : o[b][i];
                         dst = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[b][r], TS && r == 0 ? (f32x4)0.0f : dst, 0, 0, 0);
                     }
             }
             if constexpr (TS)
 #pragma unroll
-                for (int i = 0; i < 2 * NT; i++) o[0][i] += ot[i];
+                for (int b = 0; b < RB; b++)
+#pragma unroll
+                    for (int i = 0; i < 2 * NT; i++) o[b][i] += ot[b][i];
             __builtin_amdgcn_sched_barrier(0);
             if (more) issue_v(p, row_n, blk_n);
         }

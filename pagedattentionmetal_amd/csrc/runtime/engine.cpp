@@ -327,15 +327,19 @@ int32_t Context::choose_part_tokens(int64_t items_per_part, int64_t max_tiles, b
 }
 
 // Decode rows that the VALU kernel's workgroup form still serves faster than the
-// row-block kernel: f32, one query head per kv head, at most 256 tokens.  There
+// row-block kernel: f32, mostly one query head per kv head, at most 256 tokens.  There
 // the matrix form computes 16 rows for one, and a tile's f32 matrix time is the
 // longest step of the call.  Measured on gfx950 (µs per call, VALU / row blocks):
 // 8/8 d = 128: B = 4 L <= 200 9.5 / 10.1, B = 64 L <= 100 10.6 / 12.2, B = 128
 // L <= 200 26.0 / 30.8; d = 256 B = 4 L <= 200 14.1 / 17.0; 16/16 d = 64: B = 4
 // L <= 200 8.6 / 7.6, B = 64 15.7 / 16.7; 8/4 d = 128 B = 32 L <= 200 12.8 / 10.2.
+// A few rows of an odd group, one head a wave, too: 12/4 B = 4 L <= 200 d = 128 10.1 /
+// 12.1, d = 256 14.5 / 20.1, d = 64 9.1 / 8.3; d = 128 B = 64 L <= 100 19.4 / 8.7.
 static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles) {
-    return dtype == kF32 && p.num_heads == p.num_kv_heads && max_tiles <= kValuWgMaxParts &&
-           (p.head_dim > 64 || (int64_t)p.rows * p.num_heads >= 512);
+    const int64_t heads = (int64_t)p.rows * p.num_heads;
+    if (dtype != kF32 || max_tiles > kValuWgMaxParts) return false;
+    if (p.num_heads == p.num_kv_heads) return p.head_dim > 64 || heads >= 512;
+    return p.num_heads / p.num_kv_heads % 2 == 1 && p.head_dim > 64 && heads <= 64;
 }
 
 // Partition length, in 16-token tiles, of an MFMA decode that runs as partitions
@@ -1154,12 +1158,18 @@ void Context::validate_prefill(const pam_prefill_request &r) {
 // VALU / row blocks): f32 8/8 d = 128: 64 tokens 7.7 / 12.1, 32 after 200
 // 10.9 / 15.7, 64 after 100 15.1 / 16.3, 128 22.9 / 16.1; f32 16/8 d = 128: 64
 // 10.3 / 12.1, 64 after 100 20.5 / 16.7; f16 8/8 d = 96: 16 after 100 9.3 / 11.8,
-// 64 9.1 / 8.8; e4m3 8/4 d = 96: 8 tokens 9.9 / 8.3.
+// 64 9.1 / 8.8; e4m3 8/4 d = 96: 8 tokens 9.9 / 8.3; f32 12/4 d = 64: 20 tokens 6.4 /
+// 7.5, 48 6.8 / 7.7, 64 10.8 / 8.1; d = 128: 8 after 100 7.8 / 13.9, 64 12.0 / 11.9, 96
+// 12.2 / 14.8; 24/4 d = 64: 16 tokens 6.8 / 7.2, 20 7.8 / 7.4; f16 12/4 d = 96: 16 7.1 / 7.8,
+// 16 after 100 9.3 / 9.9, 48 8.9 / 8.3; f32 32/8 d = 64: 4 tokens 9.8 / 6.5.
 static bool valu_prefill_wins(const pam_layer_spec &l, int64_t rows, int64_t kv_len) {
     const int32_t G = l.num_heads / l.num_kv_heads;
     const int64_t pairs = rows * l.num_heads * kv_len;
     if (kv_len > 16 * kValuWgMaxParts || l.data_type == kFP8) return false;
-    return l.data_type == kF32 ? (G == 1 || G == 2) && pairs < 70000 : G == 1 && pairs < 31000;
+    if (l.data_type != kF32) return G % 2 == 1 && pairs < (G == 1 ? 31000 : 24000);
+    if (G <= 2) return pairs < 70000;
+    if (G % 2 == 1) return pairs < (l.head_dim > 64 ? 115000 : 48000);
+    return G % 4 == 2 && pairs < (l.head_dim > 64 ? 20000 : 9000);
 }
 
 Context::PrefillPlan Context::plan_prefill(const pam_prefill_request &r) {

@@ -35,6 +35,7 @@ def _prefill(eng, q, kd, vd, bt, T, lay, causal, off, ks=None, vs=None):
     (0, 33, 31, 8, 8, 128, 16, True, 0, 0),      # a second block of one row, a second tile of one key
     (0, 31, 1000, 8, 2, 64, 16, True, 0, 0),     # several partitions and the reduce
     (0, 70, 45, 6, 2, 80, 12, True, 0, 48),      # G = 3, head size between tiles, short partitions
+    (0, 70, 245, 6, 2, 80, 12, True, 0, 48),     # past 256 keys, where the VALU kernel no longer takes it
     (0, 5, 300, 4, 4, 256, 8, True, 0, 0),
     (0, 90, 10, 4, 1, 32, 1, False, 0, 0),       # one-token blocks, not causal
     (0, 200, 0, 4, 4, 36, 16, True, 77, 0),      # rows before the window see no key

@@ -51,7 +51,7 @@ struct PartRange {
     int nparts;
 };
 
-__device__ __forceinline__ PartRange part_range(const RowCtx &c, int part, int part_tokens) {
+__host__ __device__ __forceinline__ PartRange part_range(const RowCtx &c, int part, int part_tokens) {
     PartRange pr;
     const int tile0 = c.k_lo / 16;
     const int tile_end = (c.k_hi + 15) / 16;
@@ -61,6 +61,29 @@ __device__ __forceinline__ PartRange part_range(const RowCtx &c, int part, int p
     pr.t_begin = tile0 + part * tpp;
     pr.t_end = pr.t_begin + tpp < tile_end ? pr.t_begin + tpp : tile_end;
     return pr;
+}
+
+// A wave's contiguous share of a workgroup's tiles (possibly empty)
+__host__ __device__ __forceinline__ PartRange wave_range(const PartRange &wg, int wave, int waves) {
+    PartRange pr = wg;
+    const int per = (wg.t_end - wg.t_begin + waves - 1) / waves;
+    pr.t_begin = wg.t_begin + wave * per;
+    pr.t_end = pr.t_begin + per < wg.t_end ? pr.t_begin + per : wg.t_end;
+    return pr;
+}
+
+// Block-table entries of 64 consecutive blocks sit in one VGPR (lane i: block
+// window_blk + i).  The lane that holds token j's entry; tokens past the row's last
+// block (nlb - 1) take that block's.  A table's entries past a row's blocks may hold
+// anything, and an entry addresses the block's scales even where its keys are masked,
+// so none of them may be used (tests/native/block_window_check.cpp).
+__host__ __device__ __forceinline__ int window_lane(int j, int bsh, int window_blk, int nlb) {
+    const int blk = j >> bsh;
+    return (blk < nlb ? blk : nlb - 1) - window_blk;
+}
+// whether a window from block window_blk holds the entries of tiles below t_end
+__host__ __device__ __forceinline__ bool window_covers(int window_blk, int t_end, int bsh) {
+    return ((t_end * 16 - 1) >> bsh) - window_blk < 64;
 }
 
 // Query-head slot v of kv head kvh in row out_row.  One layer (FL false): head
@@ -222,9 +245,8 @@ __device__ __forceinline__ void mfma_core(const AttnParams &p, const RowCtx &c, 
         uint16_t ksb[kTileScale ? 1 : NI], vsb[kTileScale ? 1 : NI];
     };
 
-    // Block-table entries of 64 consecutive blocks from window_blk sit in one
-    // VGPR (lane i = block window_blk + i), refreshed once per 16-tile chunk, so
-    // a tile's address never waits on a table load.  The window covers the
+    // The window of block-table entries (window_lane) is refreshed once per 16-tile
+    // chunk, so a tile's address never waits on a table load.  It covers the
     // chunk's tiles and the tiles loaded ahead of its end.
     const int nlb = (c.k_hi + bs - 1) >> bsh;  // blocks holding keys of this row
     int window_blk = 0;
@@ -234,8 +256,9 @@ __device__ __forceinline__ void mfma_core(const AttnParams &p, const RowCtx &c, 
         const int idx = window_blk + lane < nlb ? window_blk + lane : nlb - 1;
         bt_window = c.bt[idx];
     };
-    if (early_blk >= 0 && ((pr.t_end * 16 - 1) >> bsh) - early_blk < 64) {
-        // the caller's window (blocks early_blk ..) covers every tile of this wave
+    if (early_blk >= 0 && window_covers(early_blk, pr.t_end, bsh)) {
+        // the caller's window (blocks early_blk ..) covers every tile of this wave; its
+        // lanes past the row's blocks are the table's own, which window_lane leaves out
         window_blk = early_blk;
         bt_window = early_bt;
     } else if (pr.t_begin < pr.t_end) {
@@ -256,7 +279,7 @@ __device__ __forceinline__ void mfma_core(const AttnParams &p, const RowCtx &c, 
             // offset.  Rows outside [k_lo, j_hi) read the nearest row inside
             // instead (finite data; their scores are masked to -inf, so their
             // probabilities are 0).
-            const int phys = __builtin_amdgcn_readlane(bt_window, ((lt * 16) >> bsh) - window_blk);
+            const int phys = __builtin_amdgcn_readlane(bt_window, ((lt * 16) >> bsh) - window_blk);  // a tile of keys
             const uint64_t tile_off =
                 (uint64_t)(((uint32_t)phys << bsh) + (uint32_t)((lt * 16) & (bs - 1))) * row_bytes;
             const int r_lo = c.k_lo - lt * 16 > 0 ? c.k_lo - lt * 16 : 0;
@@ -284,7 +307,7 @@ __device__ __forceinline__ void mfma_core(const AttnParams &p, const RowCtx &c, 
                 const int j = tile * 16 + trow;
                 const bool valid = j >= c.k_lo && j < j_hi;
                 const int jt = lt * 16 + trow;  // inside the window
-                const int phys = __shfl(bt_window, (jt >> bsh) - window_blk, 64);
+                const int phys = __shfl(bt_window, window_lane(jt, bsh, window_blk, nlb), 64);
                 const uint64_t off =
                     (uint64_t)(((uint32_t)phys << bsh) + (uint32_t)(jt & (bs - 1))) * row_bytes + lane_const;
                 // Every lane loads unconditionally (loads under a branch would make
@@ -453,8 +476,8 @@ __device__ __forceinline__ void mfma_item(const AttnParams &p, int r, int part, 
     const int G = slot_group<FL>(p), H = G * p.num_kv_heads;  // query-head slots
     // A decode row without a window starts at token 0, so its partitions' block-table
     // entries are requested beside the row's length (within its max_num_blocks
-    // entries; only those below the length are used): one memory latency less on a
-    // short call (1 row of 4133 tokens, 32/8 heads of 128: 9.9 -> 9.3 us).
+    // entries; mfma_core uses only those below the length): one memory latency less on
+    // a short call (1 row of 4133 tokens, 32/8 heads of 128: 9.9 -> 9.3 us).
     int early_blk = -1;
     int32_t early_bt = 0;
     if (p.mode == kRowDecode && p.window <= 0 && p.max_num_blocks > 0) {
@@ -472,13 +495,7 @@ __device__ __forceinline__ void mfma_item(const AttnParams &p, int r, int part, 
             out_head<FL, f16>(p, c.out_row, kvh, idx / HD)[idx % HD] = (f16)__builtin_nanf("");
         return;
     }
-    // this wave's contiguous share of the workgroup's tiles (possibly empty)
-    PartRange pr = wg;
-    {
-        const int per = (wg.t_end - wg.t_begin + NW - 1) / NW;
-        pr.t_begin = wg.t_begin + wave * per;
-        pr.t_end = pr.t_begin + per < wg.t_end ? pr.t_begin + per : wg.t_end;
-    }
+    const PartRange pr = wave_range(wg, wave, NW);
     float m_run, l_run;
     f32x4 o[NO];
     mfma_core<KV, HD, BLK, FL>(p, c, kvh, pr, reinterpret_cast<f16 *>(smem) + wave * WT, m_run, l_run, o,

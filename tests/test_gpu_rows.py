@@ -254,3 +254,33 @@ def test_decode_layers_partitions_bit_identical(dtype, d, lens):
         eng.decode_layers(qs, kd, vd, btd, lnd, outs, len(lens), bt.shape[1], [lay] * n, k_scale=ksd, v_scale=vsd)
         for a, b in zip(single, outs):
             assert np.array_equal(a.view(np.uint16), to_host(b).view(np.uint16))
+
+
+@pytest.mark.parametrize("H,hkv,d", [(32, 8, 128), (16, 4, 64), (32, 4, 256)])
+@pytest.mark.parametrize("lens", [[900, 5, 17, 24, 8], [1, 33, 7, 40, 16], [2003, 130]])
+def test_decode_e4m3_small_blocks_beside_other_entries(H, hkv, d, lens):
+    """e4m3 rows of 8-token blocks whose tables go on past the rows (in a wider table)
+    with a block of the pool that has scales and codes of its own: a row with an odd
+    number of blocks ends inside a 16-token tile.  Single layer and fused layers."""
+    import torch
+    bs = 8
+    rng = np.random.default_rng(82 + d + len(lens))
+    eng = _engine()
+    q, k, v, bt, lens = make_case(rng, len(lens), H, hkv, d, bs, 2, lens)
+    kd, vd, ksd, vsd, kp, vp, ks, vs = build_fp8(eng, rng, k, v, bt, lens, hkv, d, bs)
+    other = sorted(set(range(k.shape[0])) - {int(bt[b, i]) for b, L in enumerate(lens) for i in range(-(-int(L) // bs))})[0]
+    kp[other], vp[other], ks[other], vs[other] = 0x7E, 0x7E, np.inf, np.nan
+    kd, vd, ksd, vsd = to_dev(kp), to_dev(vp), to_dev(ks), to_dev(vs)
+    wide = np.full((len(lens), bt.shape[1] + 9), other, np.int32)
+    for b, L in enumerate(lens):
+        wide[b, :-(-int(L) // bs)] = bt[b, :-(-int(L) // bs)]
+    lay = layer(H, hkv, d, bs, 2)
+    ref = oracle.decode(2, q, kp, vp, wide, lens, H, k_scale=ks.view(np.uint16), v_scale=vs.view(np.uint16), n_threads=8)
+    out = torch.full(q.shape, 7.0, dtype=torch.float16, device="cuda")
+    eng.decode(to_dev(q), kd, vd, to_dev(wide), to_dev(lens), out, len(lens), wide.shape[1], lay, k_scale=ksd, v_scale=vsd)
+    assert row_rel_err(to_host(out).astype(np.float64), ref) <= TOL[2]
+    outs = [torch.full(q.shape, 7.0, dtype=torch.float16, device="cuda") for _ in range(2)]
+    eng.decode_layers([to_dev(q)] * 2, kd, vd, to_dev(wide), to_dev(lens), outs, len(lens), wide.shape[1], [lay] * 2,
+                      k_scale=ksd, v_scale=vsd)
+    for o in outs:
+        assert np.array_equal(to_host(o).view(np.uint16), to_host(out).view(np.uint16))

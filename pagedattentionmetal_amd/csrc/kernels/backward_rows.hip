@@ -116,19 +116,8 @@ struct DimOp {
     }
 };
 
-// Pool slots of the sequence's keys (-1 outside them) and their rows of one kv head
-struct KeySlots {
-    const int32_t *bt;
-    int lo, hi, bs, shift;
-    __device__ __forceinline__ KeySlots(const BackwardParams &p)
-        : bt(p.block_table), lo(p.window_start), hi(p.seq_len), bs(p.block_size), shift(block_shift(p.block_size)) {}
-    __device__ __forceinline__ int at(int j) const {
-        if (j < lo || j >= hi) return -1;
-        const int b = shift >= 0 ? j >> shift : j / bs;
-        return bt[b] * bs + (j - b * bs);
-    }
-};
-__device__ __forceinline__ const char *at_row(const char *base, int i, int64_t row_bytes, const char *zero) {
+// a row of one kv head by its pool slot (negative: the zero page)
+__device__ __forceinline__ const char *at_row(const char *base, int64_t i, int64_t row_bytes, const char *zero) {
     return i < 0 ? zero : base + i * row_bytes;
 }
 
@@ -181,9 +170,9 @@ __global__ __launch_bounds__(64 * S::W, (S::NT <= 4 ? 2 : 1)) void bwd_d_rows(Ba
     }
     const KeySlots keys(p);
     const int t1 = (p.seq_len + 15) / 16, first = p.window_start / 16 + wave;
-    auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : -1; };
+    auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : (int64_t)-1; };
     RowOp<T, S> k, v;
-    int slot = slot_of(first), ahead = slot_of(first + W);
+    int64_t slot = slot_of(first), ahead = slot_of(first + W);
     if (first < t1) {
         k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
         v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
@@ -259,9 +248,9 @@ __device__ __forceinline__ void dq_rows_body(const BackwardParams &p, int id, fl
     }
     const KeySlots keys(p);
     const int t1 = (p.seq_len + 15) / 16, first = p.window_start / 16 + wave;
-    auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : -1; };
+    auto slot_of = [&](int t) { return t < t1 ? keys.at(16 * t + n) : (int64_t)-1; };
     RowOp<T, S> k, v;
-    int slot = slot_of(first), ahead = slot_of(first + W);
+    int64_t slot = slot_of(first), ahead = slot_of(first + W);
     if (first < t1) {
         k.load(at_row(kbase, slot, kv_bytes, zero), g, d, zero);
         v.load(at_row(vbase, slot, kv_bytes, zero), g, d, zero);
@@ -322,7 +311,7 @@ __device__ __forceinline__ void dq_rows_body(const BackwardParams &p, int id, fl
 template <typename T>
 __device__ __forceinline__ void pool_add(void *pool, const BackwardParams &p, const KeySlots &keys, int j, int kvh, int e0,
                                          const float *a) {
-    T *row = static_cast<T *>(pool) + ((int64_t)keys.at(j) * p.num_kv_heads + kvh) * p.head_dim + e0;
+    T *row = static_cast<T *>(pool) + (keys.at(j) * p.num_kv_heads + kvh) * p.head_dim + e0;
     float x[4];
     load4<T>(row, x);
 #pragma unroll
@@ -345,7 +334,7 @@ __device__ __forceinline__ void dkv_rows_body(const BackwardParams &p, int id, i
     f32x4 dk[B][2 * S::NT], dv[B][2 * S::NT];
 #pragma unroll
     for (int b = 0; b < B; b++) {
-        const int slot = keys.at(key0 + 16 * b + n);
+        const int64_t slot = keys.at(key0 + 16 * b + n);
         k[b].load(at_row(static_cast<const char *>(p.k_pool) + kvh * q_bytes, slot, kv_bytes, zero), g, d, zero);
         v[b].load(at_row(static_cast<const char *>(p.v_pool) + kvh * q_bytes, slot, kv_bytes, zero), g, d, zero);
 #pragma unroll

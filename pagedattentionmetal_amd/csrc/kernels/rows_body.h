@@ -90,6 +90,27 @@ struct KPiece<uint8_t> {
     typedef f16x8 Q;
 };
 
+// A pool's token slot of token `slot` of a block: 64 bits, as a pool of narrow rows
+// holds more than 2^31 of them (tests/native/pool_slot_check.cpp)
+__host__ __device__ __forceinline__ int64_t pool_slot(int32_t block, int block_size, int slot) {
+    return (int64_t)block * block_size + slot;
+}
+
+__host__ __device__ __forceinline__ int block_shift(int bs) { return (bs & (bs - 1)) == 0 ? __builtin_ctz((unsigned)bs) : -1; }
+
+// Pool slots of a backward's sequence (-1 outside its keys)
+struct KeySlots {
+    const int32_t *bt;
+    int lo, hi, bs, shift;
+    __host__ __device__ __forceinline__ KeySlots(const BackwardParams &p)
+        : bt(p.block_table), lo(p.window_start), hi(p.seq_len), bs(p.block_size), shift(block_shift(p.block_size)) {}
+    __host__ __device__ __forceinline__ int64_t at(int j) const {
+        if (j < lo || j >= hi) return -1;
+        const int b = shift >= 0 ? j >> shift : j / bs;
+        return pool_slot(bt[b], bs, j - b * bs);
+    }
+};
+
 // The keys of a workgroup: tile t holds keys key0 + 16 t .. + 15 of the block
 // table's sequence.  Loads stay inside [lo, hi).
 struct TileKeys {
@@ -149,17 +170,17 @@ struct RowTiles {
         for (int c = 0; c < KC; c++)
             q[b][c] = *reinterpret_cast<const QOp *>(k_dim(c) < d ? (const char *)(row + k_dim(c)) : zero);
     }
-    __device__ __forceinline__ void issue_k(const AttnParams &p, int row, int block) {
+    __device__ __forceinline__ void issue_k(const AttnParams &p, int64_t row, int block) {
         const char *ptr = kbase + row * row_bytes;
         if constexpr (sizeof(KV) == 1) ks = p.k_scale[block];
 #pragma unroll
         for (int c = 0; c < KC; c++)
             k[c] = *reinterpret_cast<const KOp *>(k_dim(c) < d ? ptr + k_dim(c) * (int)sizeof(KV) : zero);
     }
-    __device__ __forceinline__ void issue_v(const AttnParams &p, int row, int block) {
+    __device__ __forceinline__ void issue_v(const AttnParams &p, int64_t row, int block) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const char *ptr = vbase + (int64_t)__shfl(row, 4 * g + r, 64) * row_bytes;
+            const char *ptr = vbase + __shfl(row, 4 * g + r, 64) * row_bytes;
             if constexpr (sizeof(KV) == 1) vs[r] = p.v_scale[__shfl(block, 4 * g + r, 64)];
 #pragma unroll
             for (int u = 0; u < NU; u++) {
@@ -183,8 +204,8 @@ struct RowTiles {
         };
         int slot, block = lookup(t0, slot), slot_n = 0, block_n = 0;
         if (t0 + step < t1) block_n = lookup(t0 + step, slot_n);
-        issue_k(p, block * bs + slot, block);
-        issue_v(p, block * bs + slot, block);
+        issue_k(p, pool_slot(block, bs, slot), block);
+        issue_v(p, pool_slot(block, bs, slot), block);
         for (int t = t0; t < t1; t += step) {
             const int kb = keys.key0 + 16 * t;
             const bool more = t + step < t1;
@@ -217,7 +238,8 @@ struct RowTiles {
             }
             __builtin_amdgcn_sched_barrier(0);
             // the next tile's K, and the block-table entry of the one after
-            const int row_n = block_n * bs + slot_n, blk_n = block_n;
+            const int64_t row_n = pool_slot(block_n, bs, slot_n);
+            const int blk_n = block_n;
             if (more) {
                 if (t + 2 * step < t1) block_n = lookup(t + 2 * step, slot_n);
                 issue_k(p, row_n, blk_n);
@@ -372,7 +394,7 @@ __device__ __forceinline__ void add_odd(const AttnParams &p, const int32_t *bt, 
     const float m_use = M == -INFINITY ? 0.0f : M;
     for (int j = j0; j < j1; j++) {
         const int blk = bt[j / bs];
-        const int64_t off = (((int64_t)blk * bs + j % bs) * p.num_kv_heads + kvh) * d;
+        const int64_t off = (pool_slot(blk, bs, j % bs) * p.num_kv_heads + kvh) * d;
         f16 ks = (f16)1.0f, vs = (f16)1.0f;
         if constexpr (sizeof(KV) == 1) ks = bits_to_f16(p.k_scale[blk]), vs = bits_to_f16(p.v_scale[blk]);
         float v[4];
@@ -392,8 +414,6 @@ __device__ __forceinline__ void add_odd(const AttnParams &p, const int32_t *bt, 
             if (!__builtin_isfinite(v[e])) a[e] += pj * v[e];
     }
 }
-
-__device__ __forceinline__ int block_shift(int bs) { return (bs & (bs - 1)) == 0 ? __builtin_ctz((unsigned)bs) : -1; }
 
 // 4 dims of a row: the result, or the row's partial for attn_reduce_kernel
 template <typename QT>

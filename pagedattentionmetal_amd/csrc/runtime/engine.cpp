@@ -439,6 +439,9 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
         const int64_t bytes = slots * ((int64_t)p.head_dim + 2) * 4;
         if (bytes >= ((int64_t)1 << 31)) throw PamError("stream-K workspace exceeds 2 GiB");
         if (fixed) {
+            if (bytes > fixed_parts) throw too_big("split-context partials", bytes, fixed_parts);
+            if (counters * 8 > (int64_t)kNoAllocCounterBytes)
+                throw too_big("merge counters", counters * 8, (int64_t)kNoAllocCounterBytes);
             p.part_o = reinterpret_cast<float *>(fixed + kNoAllocZeroBytes + kNoAllocCounterBytes);
             p.seg_count = reinterpret_cast<uint64_t *>(fixed + kNoAllocZeroBytes);
         } else {

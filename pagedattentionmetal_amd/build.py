@@ -22,9 +22,9 @@ ARCH = "gfx950"
 # Packed FP32 VALU forms are disabled for all device code; hipcc's host pass
 # warns that it does not know the feature, which is harmless.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-# per-source additions: the backward kernels keep their MFMA results in VGPRs
+# per-source additions: the backward and row-block kernels keep their MFMA results in VGPRs
 # (with the default AGPR form the compiler copies every score tile out of AGPRs)
-FILE_FLAGS = {"backward.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("backward.hip", "rows.hip")}
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"--offload-arch={ARCH}",
           "-fvisibility=hidden"]
 

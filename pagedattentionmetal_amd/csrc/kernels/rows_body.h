@@ -12,6 +12,14 @@
 // O^T += V^T P^T over the keys {r, 4 + r, 8 + r, 12 + r} on
 // v_mfma_f32_16x16x4_f32.  Probabilities, sums and outputs stay in f32 registers.
 //
+// Sums of f32 caches: a score adds up in a tree (dot_tree), a tile's outputs by
+// themselves before they join the row's.  Error norms against 64 bits over those of
+// the VALU rows (which add a lane's 4 products and then lanes, pairwise), geometric
+// mean and largest of 30 to 60 calls a head size: decode 0.87-0.93 and 1.05-1.16 (a few
+// outputs of one row), prefill 0.66-0.90 and 1.03.  With one chain of a tile's outputs
+// and two to eight chains of a score: 0.96-1.06 and 1.23, 0.80-1.07 and 1.40.  Time
+// against that: prefills of 2048 tokens 2-5% more, short ones 4-11%, decodes 2-5%.
+//
 // Operands come straight from the pools: a lane loads its K operand in 16-byte
 // pieces (a key's 64 bytes per instruction) and its V operand as VW consecutive
 // dims of one key (whole 256-byte rows per instruction at d = 128), one tile
@@ -24,8 +32,8 @@
 // is 2048 matrix cycles for 16 KB in f32, 1150 for 8 KB in f16), and, for e4m3,
 // the f32 matrix time of O^T.  Measured on gfx950 against the VALU rows that
 // served these calls before (µs per call): f32 8/8 d = 128, 777 tokens after 391
-// 784 -> 54 (45 TFLOP/s); f32 32/8 d = 128, 2048 tokens 379 (91 TFLOP/s); f16
-// 32/8 d = 96, 2048 tokens 166 (155 TFLOP/s); f16 16/16 d = 64 decode of 24 rows
+// 784 -> 55 (44 TFLOP/s); f32 32/8 d = 128, 2048 tokens 399 (86 TFLOP/s); f16
+// 32/8 d = 96, 2048 tokens 162 (159 TFLOP/s); f16 16/16 d = 64 decode of 24 rows
 // of up to 3000 tokens 162 -> 48 (3.4 TB/s); f32 8/8 d = 128 64 rows of up to
 // 2000 128 -> 117 (4.9 TB/s); f32 32/8 one row of 5598 337 -> 12; e4m3 12/4
 // d = 128 205 rows of up to 4000 2620 -> 172.
@@ -120,6 +128,56 @@ struct TileKeys {
     int block_size, shift;  // shift: log2(block_size), or -1
 };
 
+// The compiler otherwise moves additions whose results are read later down to there,
+// and every product summed by them holds its registers until then.
+__device__ __forceinline__ void keep_here(f32x4 &x) { asm volatile("" : "+v"(x)); }
+
+// f32 products of 16 rows a and 16 columns b over KC pieces of 16 dims (4 a lane).
+// The matrix unit sums LEAF dims, and these sums add up in a tree, as the VALU kernels
+// add a lane's 4 products and then the lanes.  The additions of a piece follow the
+// products of the next, which hide them.
+template <int LEAF, int KC>
+__device__ __forceinline__ f32x4 dot_tree(const f32x4 (&a)[KC], const f32x4 (&b)[KC]) {
+    constexpr int T = 16 / LEAF;  // leaves of a piece
+    f32x4 t[2][T], level[8];
+    // the additions of piece c, in the order in which its products end
+    auto add = [&](int c, int step) {
+        f32x4 *x = t[c & 1];
+        if (T == 4 && step < 2) {
+            x[step] += x[step + 2];
+            keep_here(x[step]);
+        } else if (step == 2) {
+            x[0] += x[1];
+            keep_here(x[0]);
+        } else if (step == 3) {
+            int l = 0;
+#pragma unroll
+            for (; (c >> l) & 1; l++) x[0] += level[l];
+            level[l] = x[0];
+            keep_here(level[l]);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            f32x4 &x = t[c & 1][e % T];
+            x = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c][e], b[c][e], e < T ? (f32x4)0.0f : x, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (c) add(c - 1, e);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+    for (int e = 0; e < 4; e++) add(KC - 1, e);
+    f32x4 s = (f32x4)0.0f;
+    bool any = false;
+#pragma unroll
+    for (int l = 0; l < 8; l++)
+        if ((KC >> l) & 1) s = any ? s + level[l] : level[l], any = true;
+    keep_here(s);
+    return s;
+}
+
 template <typename KV, typename QT, int NT, int RB>
 struct RowTiles {
     static constexpr bool F32 = sizeof(KV) == 4;
@@ -129,6 +187,7 @@ struct RowTiles {
     static constexpr int VW = F32 ? (NT % 2 == 0 ? 4 : 2) : (NT % 4 == 0 ? 8 : (NT == 2 ? 4 : 2));
     static constexpr int NU = 2 * NT / VW;
     static constexpr int LS = 32 * NT + 4;           // LDS row stride (floats)
+    static constexpr int LEAF = RB > 1 && NT > 3 ? 8 : 4;  // dot_tree's, as the registers allow
     typedef typename KPiece<KV>::K KOp;
     typedef typename KPiece<KV>::Q QOp;
 
@@ -209,31 +268,22 @@ struct RowTiles {
         for (int t = t0; t < t1; t += step) {
             const int kb = keys.key0 + 16 * t;
             const bool more = t + step < t1;
-            // f32: the scores in several chains of sums, added pairwise, for less
-            // rounding than one long chain; as many as the registers hold
-            constexpr int CH = F32 ? (RB > 1 ? (NT <= 2 ? 4 : 2) : (NT >= 4 ? 8 : 4)) : 1;
-            f32x4 s[RB], sc[RB][CH];
+            f32x4 s[RB];
+            if constexpr (F32) {
 #pragma unroll
-            for (int b = 0; b < RB; b++)
+                for (int b = 0; b < RB; b++) s[b] = dot_tree<LEAF, KC>(k, q[b]);
+            } else {
 #pragma unroll
-                for (int i = 0; i < CH; i++) sc[b][i] = (f32x4)0.0f;
+                for (int b = 0; b < RB; b++) s[b] = (f32x4)0.0f;
 #pragma unroll
-            for (int c = 0; c < KC; c++) {
-                if constexpr (F32) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-#pragma unroll
-                        for (int b = 0; b < RB; b++)
-                            sc[b][(4 * c + e) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[b][c][e], sc[b][(4 * c + e) % CH], 0, 0, 0);
-                } else {
+                for (int c = 0; c < KC; c++) {
                     f16x8 a;
                     if constexpr (sizeof(KV) == 1)
                         a = e4m3x8_dequant(k[c][0], k[c][1], bits_to_f16(ks));
                     else
                         a = k[c];
 #pragma unroll
-                    for (int b = 0; b < RB; b++)
-                        sc[b][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[b][c], sc[b][0], 0, 0, 0);
+                    for (int b = 0; b < RB; b++) s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q[b][c], s[b], 0, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -245,14 +295,6 @@ struct RowTiles {
                 issue_k(p, row_n, blk_n);
             }
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int b = 0; b < RB; b++) {
-#pragma unroll
-                for (int h = CH / 2; h > 0; h /= 2)
-#pragma unroll
-                    for (int i = 0; i < h; i++) sc[b][i] += sc[b][i + h];
-                s[b] = sc[b][0];
-            }
             // Online softmax.  The reference max of a row moves only when a score
             // passes it by 8, a factor of 2^8 (or the row has none yet): the probabilities
             // are f32, so their scale is free, and most tiles need no reduction across
@@ -295,49 +337,63 @@ struct RowTiles {
                     l[b] += s[b][r];
                 }
             }
-            // f32, where the registers hold it: a tile's O^T is summed by itself and then
-            // added, which shortens the chains of sums.  Error against 64 bits, VALU rows
-            // / one chain of outputs and two of scores / this: decode 32/8 d = 64, 64
-            // rows of up to 500 tokens 1.24e-7 / 1.66e-7 / 1.30e-7; 8/8 d = 128, 16 rows
-            // of up to 600 1.60e-7 / 1.71e-7 / 1.30e-7; 32/8 d = 128, 4000 tokens 3.1e-7 /
-            // 1.8e-7 / 1.6e-7; up to 100 tokens 1.03e-7 / 1.3e-7 / 1.1e-7 (an f32 ulp is
-            // 1.2e-7); prefill d = 64 32/8, 874 tokens 1.14e-7 / 1.37e-7 / 1.05e-7, 8/8,
-            // 777 after 391 1.86e-7 / 2.14e-7 / 1.49e-7.  Times (µs per call, without /
-            // with): those decodes the same; the prefills 51 / 58 (554 on the VALU rows)
-            // and 33 / 33, 8/2 2048 tokens 84 / 82.
-            constexpr bool TS = F32 && NT <= (RB == 1 ? 4 : 2);
-            f32x4 ot[RB][TS ? 2 * NT : 1];
             // O^T.  In an edge tile a V element of a key that some row must not see
             // enters only if it is finite (0 * Inf would reach the rows that mask
             // it); add_odd gives the others to the rows that do see the key.
+            auto hide = [&](int r, float &x) {
+                const int j = kb + 4 * g + r;
+                const bool bad = !(j >= keys.lo && j < keys.hi_all) && !__builtin_isfinite(x);
+                odd |= bad;
+                x = bad ? 0.0f : x;
+            };
+            if constexpr (F32) {
+                if (!full)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                float a[2 * NT];
+                    for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int u = 0; u < NU; u++) v[r][u].floats(sizeof(KV) == 1 ? vs[r] : (uint16_t)0, a + VW * u);
-                if (!full) {
-                    const int j = kb + 4 * g + r;
-                    const bool all = j >= keys.lo && j < keys.hi_all;
+                        for (int i = 0; i < 2 * NT; i++) {
+                            float x = v[r][i / VW].v[i % VW];
+                            hide(r, x);
+                            v[r][i / VW].v[i % VW] = x;
+                        }
+                // A tile's sum by itself, in two chains of 8 keys, then added; the additions
+                // follow the next sum's products, as in dot_tree.
+                constexpr int N = 2 * NT * RB;
+                f32x4 t[2][2];
+                auto add = [&](int x, int step) {
+                    f32x4 *y = t[x & 1], &sum = o[x % RB][x / RB];
+                    if (step == 2) y[0] += y[1], keep_here(y[0]);
+                    if (step == 3) sum += y[0], keep_here(sum);
+                };
 #pragma unroll
-                    for (int i = 0; i < 2 * NT; i++) {
-                        const bool bad = !all && !__builtin_isfinite(a[i]);
-                        odd |= bad;
-                        a[i] = bad ? 0.0f : a[i];
+                for (int x = 0; x < N; x++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int i = x / RB;
+                        f32x4 &y = t[x & 1][r & 1];
+                        y = __builtin_amdgcn_mfma_f32_16x16x4f32(v[r][i / VW].v[i % VW], s[x % RB][r],
+                                                                 r < 2 ? (f32x4)0.0f : y, 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (x) add(x - 1, r);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                add(N - 1, 2), add(N - 1, 3);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float a[2 * NT];
+#pragma unroll
+                    for (int u = 0; u < NU; u++) v[r][u].floats(sizeof(KV) == 1 ? vs[r] : (uint16_t)0, a + VW * u);
+                    if (!full)
+#pragma unroll
+                        for (int i = 0; i < 2 * NT; i++) hide(r, a[i]);
+#pragma unroll
+                    for (int i = 0; i < 2 * NT; i++)
+#pragma unroll
+                        for (int b = 0; b < RB; b++)
+                            o[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[b][r], o[b][i], 0, 0, 0);
                 }
-#pragma unroll
-                for (int i = 0; i < 2 * NT; i++)
-#pragma unroll
-                    for (int b = 0; b < RB; b++) {
-                        f32x4 &dst = TS ? ot[b][i] : o[b][i];
-                        dst = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], s[b][r], TS && r == 0 ? (f32x4)0.0f : dst, 0, 0, 0);
-                    }
             }
-            if constexpr (TS)
-#pragma unroll
-                for (int b = 0; b < RB; b++)
-#pragma unroll
-                    for (int i = 0; i < 2 * NT; i++) o[b][i] += ot[b][i];
             __builtin_amdgcn_sched_barrier(0);
             if (more) issue_v(p, row_n, blk_n);
         }

@@ -284,3 +284,62 @@ def test_decode_e4m3_small_blocks_beside_other_entries(H, hkv, d, lens):
                       k_scale=ksd, v_scale=vsd)
     for o in outs:
         assert np.array_equal(to_host(o).view(np.uint16), to_host(out).view(np.uint16))
+
+
+def _attend64(q, k, v, lens):
+    """float64 attention of rows q [n, H, d], row i over the first lens[i] of its keys k[i], v[i] [L, hkv, d]."""
+    out = np.empty(q.shape)
+    G = q.shape[1] // k[0].shape[1]
+    for i, L in enumerate(lens):
+        kk, vv = (np.repeat(x[i][:L].astype(np.float64), G, axis=1) for x in (k, v))
+        s = np.einsum("hd,jhd->hj", q[i].astype(np.float64), kk) / np.sqrt(q.shape[2])
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[i] = np.einsum("hj,jhd->hd", p / p.sum(1, keepdims=True), vv)
+    return out
+
+
+def _norm_err(a, ref):
+    return np.linalg.norm(a.astype(np.float64) - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("H,hkv,d,T,off", [(64, 8, 128, 101, 0), (16, 4, 128, 143, 0), (32, 2, 96, 40, 300),
+                                           (8, 4, 256, 90, 20)])
+def test_rows_f32_prefill_error_against_the_valu_kernel(H, hkv, d, T, off):
+    """The matrix units' f32 sums are no further from 64 bits than the VALU kernel's
+    (a ratio of error norms over tens of thousands of outputs moves by 1% with the
+    inputs; 3% allowed)."""
+    bs, err = 16, {0: 0.0, 1: 0.0}
+    for seed in range(3):
+        rng = np.random.default_rng(500 + seed)
+        _, k, v, bt, _ = make_case(rng, 1, H, hkv, d, bs, 0, [off + T])
+        k, v = 0.5 * k, 0.5 * v
+        q = rng.standard_normal((T, H, d)).astype(np.float32)
+        kr, vr = (x[bt[0]].reshape(-1, hkv, d) for x in (k, v))
+        ref = _attend64(q, [kr] * T, [vr] * T, [off + i + 1 for i in range(T)])
+        for choice in err:
+            eng = _engine()
+            eng.set_decode_kernel(choice)
+            err[choice] += _norm_err(_prefill(eng, q, to_dev(k), to_dev(v), bt[0], T, layer(H, hkv, d, bs, 0), True, off), ref)
+    assert err[0] <= 1.03 * err[1], err
+
+
+@pytest.mark.parametrize("H,hkv,d,B,hi", [(8, 1, 256, 49, 244), (8, 1, 128, 40, 69), (32, 8, 64, 64, 36), (32, 8, 256, 29, 191)])
+def test_rows_f32_decode_error_against_the_valu_kernel(H, hkv, d, B, hi):
+    """As above, short decodes (fewer outputs: 5%)."""
+    import torch
+    bs, err = 16, {0: 0.0, 1: 0.0}
+    for seed in range(3):
+        rng = np.random.default_rng(600 + seed)
+        lens = rng.integers(hi // 4, hi + 1, B)
+        lens[0] = hi
+        q, k, v, bt, lens = make_case(rng, B, H, hkv, d, bs, 0, lens)
+        k, v = 0.5 * k, 0.5 * v
+        rows = lambda x: [x[bt[i]].reshape(-1, hkv, d) for i in range(B)]
+        ref = _attend64(q, rows(k), rows(v), [int(L) for L in lens])
+        for choice in err:
+            eng = _engine()
+            eng.set_decode_kernel(choice)
+            out = torch.full(q.shape, 7.0, dtype=torch.float32, device="cuda")
+            eng.decode(to_dev(q), to_dev(k), to_dev(v), to_dev(bt), to_dev(lens), out, B, bt.shape[1], layer(H, hkv, d, bs, 0))
+            err[choice] += _norm_err(to_host(out), ref)
+    assert err[0] <= 1.05 * err[1], err

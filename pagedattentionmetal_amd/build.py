@@ -24,7 +24,7 @@ ARCH = "gfx950"
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # per-source additions: the backward and row-block kernels keep their MFMA results in VGPRs
 # (with the default AGPR form the compiler copies every score tile out of AGPRs)
-FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("backward.hip", "rows.hip")}
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("backward.hip", "backward_rows.hip", "rows.hip")}
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"--offload-arch={ARCH}",
           "-fvisibility=hidden"]
 

@@ -18,16 +18,22 @@
 // lane, in two forms: as rows (lane n's row, a piece of its dims) for S and dP,
 // and by dims (VW dims of one row) for the gradients.
 //
+// Sums of f32 caches: S and dP add up in a tree (dot_tree).  Error norms of the
+// gradients against 64 bits over the VALU kernels', geometric mean of 45 to 57 calls a
+// head size: 0.45-0.63, largest 1.02.  With two chains over the head: 0.48-0.74, and up to
+// 1.84 for a few tokens; the tree costs 2-4% of a call up to d = 128 (MFMA results in VGPRs
+// take 10% off at d = 256).
+//
 // What bounds it: the f32 matrix rate (nine products over the (row, key) pairs
 // where five are needed: S and dP are formed for D, for dQ and for dK / dV); a
 // short sequence, its few workgroups and the latency of its tiles' loads.  Measured
 // on gfx950 against the VALU kernels, which served these shapes before (µs per
-// call): f32 8/2 d = 64, 600 tokens 2500 -> 78 (D 21, gradients 52, sum 5); f32 16/4
-// d = 64, 1000 tokens 7160 -> 247; f16 8/8 d = 64, 1000 tokens 3700 -> 77; f16 32/8
-// d = 64, 2000 tokens 50300 -> 847 (97 TFLOP/s of the five products).  One block of
-// rows or keys a wave in place of two: 322, 106 and 1124 for the last three; D alone
-// with one: 259, 83 and 940.  dQ (with D) and dK / dV in launches of their own, where
-// each leaves CUs idle: 94, 246, 76 and 858; 12/4 d = 96, 200 tokens 50 against 40.
+// call): f32 8/2 d = 64, 600 tokens 2500 -> 80; f32 16/4 d = 64, 1000 tokens 7160 -> 235;
+// f16 8/8 d = 64, 1000 tokens 3700 -> 77; f16 32/8 d = 64, 2000 tokens 50300 -> 847 (97
+// TFLOP/s of the five products).  One block of rows or keys a wave in place of two:
+// 322, 106 and 1124 for the last three; D alone with one: 259, 83 and 940.  dQ (with D)
+// and dK / dV in launches of their own, where each leaves CUs idle: 94, 246, 76 and 858;
+// 12/4 d = 96, 200 tokens 50 against 40.  f32 32/8 d = 128, 1000 tokens: 1091 (38 TFLOP/s).
 #include "rows_body.h"
 
 namespace pam {
@@ -64,23 +70,16 @@ struct RowOp {
             v[c] = *reinterpret_cast<const V *>(S::EX || e < d ? row + e * (int)sizeof(T) : zero);
         }
     }
-    // 16x16 products of rows a (the result's rows) and b (its columns); f32 in two
-    // chains of sums, which halves the chains' rounding
+    // 16x16 products of rows a (the result's rows) and b (its columns)
     __device__ __forceinline__ static f32x4 dot(const RowOp &a, const RowOp &b) {
-        f32x4 s = (f32x4)0.0f, s2 = (f32x4)0.0f;
+        if constexpr (sizeof(T) == 4) {
+            return dot_tree<8, S::KC>(a.v, b.v);
+        } else {
+            f32x4 s = (f32x4)0.0f;
 #pragma unroll
-        for (int c = 0; c < S::KC; c++) {
-            if constexpr (sizeof(T) == 4) {
-#pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[c][e], b.v[c][e], s, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[c][e + 1], b.v[c][e + 1], s2, 0, 0, 0);
-                }
-            } else {
-                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v[c], b.v[c], s, 0, 0, 0);
-            }
+            for (int c = 0; c < S::KC; c++) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v[c], b.v[c], s, 0, 0, 0);
+            return s;
         }
-        return sizeof(T) == 4 ? s + s2 : s;
     }
 };
 

@@ -74,3 +74,33 @@ def test_backward_refuses_fp8(torch_mod=None):
     x = torch.zeros(64, device="cuda")
     with pytest.raises(PagedAttentionError, match="f32 or f16"):
         eng.backward(x, x, x, x, x, x, x, x, x, x, 4, PagedLayerSpec(16, 2, 2, 16, 2))
+
+
+@pytest.mark.parametrize("H,hkv,d,T", [(32, 32, 256, 19), (12, 4, 96, 26), (8, 1, 64, 33), (16, 4, 128, 70)])
+def test_backward_f32_error_against_the_valu_kernels(H, hkv, d, T):
+    """The f32 matrix kernels' gradients are no further from 64 bits than those of the
+    VALU kernels, which take buffers that are not 16-byte aligned (5% for what the
+    ratio of the error norms moves with the inputs)."""
+    import torch
+    from pagedattentionmetal_amd import PagedAttentionEngine, PagedLayerSpec
+    bs, err = 16, np.zeros((2, 3))
+    shifted = lambda a: torch.cat([torch.zeros(1, device="cuda"), to_dev(a).reshape(-1)])[1:].view(a.shape)
+    for seed in range(3):
+        rng = np.random.default_rng(700 + seed)
+        nbl = (T + bs - 1) // bs
+        bt = rng.permutation(nbl).astype(np.int32)
+        kp, vp = (0.5 * rng.standard_normal((nbl, bs, hkv, d)).astype(np.float32) for _ in range(2))
+        q, go = (rng.standard_normal((T, H, d)).astype(np.float32) for _ in range(2))
+        m, l, _ = oracle.forward_stats(q, kp, vp, bt, window=0)
+        m, l = m.astype(np.float32), l.astype(np.float32)
+        ref = oracle.backward(q, kp, vp, bt, go, m, l, window=0)
+        slots = (bt[np.arange(T) // bs], np.arange(T) % bs)
+        for i, put in enumerate((to_dev, shifted)):
+            eng = PagedAttentionEngine()
+            eng.set_graceful_degradation(False)
+            dq, dkp, dvp = torch.zeros((T, H, d), device="cuda"), to_dev(np.zeros_like(kp)), to_dev(np.zeros_like(vp))
+            eng.backward(put(q), to_dev(kp), to_dev(vp), to_dev(bt), to_dev(go), to_dev(m), to_dev(l), dq, dkp, dvp, T,
+                         PagedLayerSpec(d, H, hkv, bs, 0, 0))
+            for x, (a, b) in enumerate(zip((to_host(dq), to_host(dkp)[slots], to_host(dvp)[slots]), ref)):
+                err[i, x] += np.linalg.norm(a.astype(np.float64) - b) / np.linalg.norm(b)
+    assert (err[0] <= 1.05 * err[1]).all(), err

@@ -358,18 +358,39 @@ static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles)
 // rows L = 1000 26.0 / 16.7, L = 4000 37.8 / 45.8, 128 rows L = 500 33.2 / 24.7, L =
 // 1000 40.1 / 41.4; f16 d = 64: 32 rows L = 1000 21.3 / 11.4; d = 256 (64/8): 32 rows
 // L = 1000 47.5 / 33.0, 128 rows L = 500 77.5 / 75.1, 256 rows L = 200 74.1 / 93.8.
-static int64_t mfma_part_tiles(int64_t pairs, int64_t max_tiles, int32_t head_dim, int32_t dtype, int32_t cus) {
+//
+// The lengths above are of tables as wide as the longest row.  Rows that end early in a
+// wide table leave the chip to the few partitions before their end, so few pairs keep
+// partitions short whatever the table's width: up to 8 pairs as few_part_tiles has them, up
+// to 16 pairs 512 tokens.  700 decodes, tables of 1 to 16 times the longest row: 24 -> 11
+// slower by 5% or more than stream-K or 256-token partitions, at most 1.38x -> 1.23x (µs: 9
+// rows L <= 5800 in 23000 d = 256 28.4 -> 21.7; 11 rows L = 2900 in 46000 e4m3 d = 64 23.1
+// -> 12.3), 0.7% less time on average; 3 slower by 16% to 26% (1 row of 13700 d = 256 33.8 ->
+// 39.2).
+//
+// Prefill rows all reach the table's end, so at d > 128, one workgroup a CU, they take one
+// round (µs: 67 rows 8/1 e4m3, 8-token blocks, 3800 keys 317 -> 193).
+static int64_t few_part_tiles(int64_t pairs, int64_t max_tiles, int32_t cus) {
+    int64_t t = 64;
+    while (t > 16 && pairs * ceil_div(max_tiles, t) < 3 * (int64_t)cus) t /= 2;
+    return t;
+}
+static int64_t mfma_part_tiles(int64_t pairs, int64_t max_tiles, int32_t head_dim, int32_t dtype, bool prefill,
+                               int32_t cus) {
     if (max_tiles <= 0) return 0;
     const int64_t row_bytes = std::min<int64_t>(2 * (int64_t)head_dim * elem_bytes(dtype), 512);
+    const int64_t few = few_part_tiles(pairs, max_tiles, cus);
     if (pairs * max_tiles * 16 * row_bytes <= 150000000) {
         if (max_tiles <= (head_dim > 128 ? 16 : 32)) return max_tiles;
         int64_t t = 8;
         while (t < 32 && t * 32 < max_tiles) t *= 2;  // at most 32 partials to merge, up to 512 tokens
         // e4m3, whose workgroups wait on their widening more than on memory, up to
         // 1.5 a CU (3 rows L = 4000: 14.6 at 256 tokens, 16.5 at 512; f16 21.1, 18.3)
-        const int64_t most = dtype == kFP8 ? cus + cus / 2 : cus + cus / 4;
+        int64_t most = dtype == kFP8 ? cus + cus / 2 : cus + cus / 4;
+        if (prefill && head_dim > 128) most = cus;
         while (t < max_tiles && pairs * ceil_div(max_tiles, t) > most) t *= 2;
         t = std::min(t, max_tiles);
+        if (pairs <= 16) t = std::min(t, pairs <= 8 ? few : 32);
         // a workgroup's own stream must stay short: 1024 tokens, or 2048 where
         // that is the whole row or there are few pairs
         if (t <= 64 || (t <= 128 && (t == max_tiles || pairs <= 64))) return t;
@@ -377,12 +398,7 @@ static int64_t mfma_part_tiles(int64_t pairs, int64_t max_tiles, int32_t head_di
     // few pairs of long rows: units of one pair would merge one batch after
     // another (µs per call, stream-K / 256-token partitions: 1 row 64K tokens 87.6 /
     // 65.9, 2 rows 16K 49.2 / 44.0; 2 rows 64K 99.1 / 103.2)
-    if (pairs <= 8 || (pairs <= 16 && max_tiles <= 2048)) {
-        int64_t t = 64;
-        while (t > 16 && pairs * ceil_div(max_tiles, t) < 3 * (int64_t)cus) t /= 2;
-        return t;
-    }
-    return 0;
+    return pairs <= 8 || (pairs <= 16 && max_tiles <= 2048) ? few : 0;
 }
 
 // Split-context set-up of a row launch (p.rows and the shape already filled).
@@ -429,7 +445,9 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
             throw too_big("merge counters", count * 8, (int64_t)kNoAllocCounterBytes);
     }
     int64_t part_tiles =
-        use_mfma && part_tokens_override == 0 ? mfma_part_tiles(pairs, max_tiles, p.head_dim, dtype, cus_) : 0;
+        use_mfma && part_tokens_override == 0
+            ? mfma_part_tiles(pairs, max_tiles, p.head_dim, dtype, p.mode == kRowPrefill, cus_)
+            : 0;
     if (fixed && part_tiles > 0 && part_tiles < max_tiles &&
         p.rows * (int64_t)p.num_heads * ceil_div(max_tiles, part_tiles) * (p.head_dim + 2) * 4 > fixed_parts)
         part_tiles = 0;

@@ -343,3 +343,39 @@ def test_rows_f32_decode_error_against_the_valu_kernel(H, hkv, d, B, hi):
             eng.decode(to_dev(q), to_dev(k), to_dev(v), to_dev(bt), to_dev(lens), out, B, bt.shape[1], layer(H, hkv, d, bs, 0))
             err[choice] += _norm_err(to_host(out), ref)
     assert err[0] <= 1.05 * err[1], err
+
+
+def _wide(bt, pool, width):
+    """Tables widened to `width` blocks, and a pool that may hold them (a call checks that)."""
+    w = np.zeros((bt.shape[0], width), np.int32)
+    w[:, :bt.shape[1]] = bt
+    need = max(0, w.size - pool.shape[0])
+    return w, np.concatenate([pool, np.zeros((need,) + pool.shape[1:], pool.dtype)])
+
+
+@pytest.mark.parametrize("dtype,H,hkv,d,B,width,most", [
+    (1, 8, 1, 256, 9, 1456, 512),    # 9 to 16 pairs: 512 tokens
+    (2, 16, 4, 64, 3, 1500, 512),
+    (1, 32, 2, 128, 3, 1984, 256),   # up to 8 pairs: 256 while a CU has no three partitions
+    (2, 8, 1, 256, 4, 772, 256),
+])
+def test_mfma_decode_of_few_pairs_keeps_short_partitions(dtype, H, hkv, d, B, width, most):
+    """Tables much wider than their rows (blocks of 16)."""
+    import torch
+    rng = np.random.default_rng(86)
+    eng = _engine()
+    q, k, v, bt, lens = make_case(rng, B, H, hkv, d, 16, dtype, rng.integers(100, 700, B))
+    if dtype == 2:
+        kd, vd, ksd, vsd, k, v, ks, vs = build_fp8(eng, rng, k, v, bt, lens, hkv, d, 16)
+        ks, vs = ks.view(np.uint16), vs.view(np.uint16)
+    else:
+        ks = vs = None
+    bw, kp = _wide(bt, k, width)
+    kd, vd = to_dev(kp), to_dev(_wide(bt, v, width)[1])
+    ksd, vsd = (None, None) if ks is None else (to_dev(np.resize(x, kp.shape[0]).view(np.float16)) for x in (ks, vs))
+    out = torch.full(q.shape, 7.0, dtype=torch.float16, device="cuda")
+    eng.decode(to_dev(q), kd, vd, to_dev(bw), to_dev(lens), out, B, width, layer(H, hkv, d, 16, dtype), k_scale=ksd, v_scale=vsd)
+    parts = eng.last_stats["temporary_bytes"] // (B * H * (d + 2) * 4)
+    assert parts >= -(-width * 16 // most)
+    ref = oracle.decode(dtype, q, k, v, bw, lens, H, k_scale=ks, v_scale=vs, n_threads=8)
+    assert row_rel_err(to_host(out).astype(np.float64), ref) <= TOL[dtype]

@@ -353,6 +353,37 @@ def _wide(bt, pool, width):
     return w, np.concatenate([pool, np.zeros((need,) + pool.shape[1:], pool.dtype)])
 
 
+@pytest.mark.parametrize("H,hkv,d,lens,width,valu", [
+    (4, 4, 256, [250, 3, 64], 32, True),      # one head a kv head, d > 128: up to 512 tokens
+    (4, 4, 256, [250, 3, 64], 33, False),
+    (4, 4, 256, [300] * 33, 24, True),        # more heads: up to 384
+    (4, 4, 256, [300] * 33, 25, False),
+    (8, 8, 128, [190, 40], 24, True),         # few heads: up to 384
+    (8, 8, 128, [190, 40], 25, False),
+    (8, 8, 128, [190] * 9, 24, False),
+    (12, 4, 256, [177, 20], 24, True),        # an odd group
+    (12, 4, 96, [177, 20], 24, True),
+    (12, 4, 96, [177, 20] * 3, 24, False),
+    (8, 4, 256, [177, 20], 16, False),        # an even group
+])
+def test_f32_decode_rows_of_few_keys_stay_on_the_valu_kernel(H, hkv, d, lens, width, valu):
+    """By the table's width, in blocks of 16: the same bits as with set_decode_kernel(1)."""
+    import torch
+    rng = np.random.default_rng(85)
+    q, k, v, bt, lens = make_case(rng, len(lens), H, hkv, d, 16, 0, lens)
+    bw, k = _wide(bt, k, width)
+    _, v = _wide(bt, v, width)
+    got = []
+    for choice in (0, 1):
+        eng = _engine()
+        eng.set_decode_kernel(choice)
+        out = torch.full(q.shape, 7.0, dtype=torch.float32, device="cuda")
+        eng.decode(to_dev(q), to_dev(k), to_dev(v), to_dev(bw), to_dev(lens), out, len(lens), width, layer(H, hkv, d, 16, 0))
+        got.append(to_host(out))
+    assert row_rel_err(got[0].astype(np.float64), oracle.decode(0, q, k, v, bw, lens, H, n_threads=8)) <= TOL[0]
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)) == valu
+
+
 @pytest.mark.parametrize("dtype,H,hkv,d,B,width,most", [
     (1, 8, 1, 256, 9, 1456, 512),    # 9 to 16 pairs: 512 tokens
     (2, 16, 4, 64, 3, 1500, 512),

@@ -91,10 +91,13 @@ struct AttnParams {
     uint32_t epoch;
     // VALU kernel: 1 runs a (row, head group)'s partitions as the waves of one
     // workgroup (attn_valu_wg_kernel), merged in LDS
-    int32_t valu_wg;
+    int16_t valu_wg;
     // 1: the row-block kernels (rows.hip) in place of the VALU kernel
-    int32_t row_blocks;
+    int16_t row_blocks;
 };
+// A kernel's second argument follows at 312 bytes, in the parameters' last 64-byte line:
+// one more field moved it to a line of its own and cost a short VALU decode 0.06 µs.
+static_assert(sizeof(AttnParams) <= 312, "AttnParams");
 
 // Entry points of a loaded code object (libpam_kernels.hsaco, module_entry.hip).
 // A launcher given a table launches a configuration the table holds through

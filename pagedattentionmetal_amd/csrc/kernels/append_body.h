@@ -41,8 +41,10 @@ __device__ __forceinline__ void append_body(const AppendParams &p, int64_t chunk
 // that is exactly half way goes to the larger magnitude; raising every quotient by
 // 2^-20 therefore leaves the nearest code as it is, ties included, and the IEEE
 // division with its case analysis becomes a product, an add and a shift.
-// (test_fp8_fast_quantiser checks all 2^31 pairs of halves.)
+// (test_fp8_fast_quantiser checks all 2^31 pairs of halves on the CPU; contraction is off,
+// as the device would otherwise fuse the product with the sum below it.)
 __host__ __device__ __forceinline__ uint32_t fp8_code(float v, float inv) {
+#pragma clang fp contract(off)
     const float x = __builtin_fabsf(v) * inv;
     const uint32_t b = __builtin_bit_cast(uint32_t, x);
     uint32_t normal = ((b + 0x80000u) >> 20) - (120u << 3);  // 3-bit mantissa, half away from zero

@@ -489,9 +489,10 @@ int64_t Context::plan_split(AttnParams &p, int32_t dtype, bool use_mfma, int64_t
     if (!use_mfma && p.mode != kRowPrefill && decode_kernel_choice != 1 && rows_supported(p, dtype) &&
         p.rows <= kMaxGridYZ && !valu_rows_win(p, dtype, max_tiles)) {
         // Row-block kernel: one workgroup per (row, slot of up to 16 heads,
-        // partition).  A row is cut until there are about 8 workgroups per CU, to
-        // no less than 256 tokens (a partition's start and the reduce cost more
-        // than they spread), or 128 for few pairs with long contexts.  Measured on
+        // partition).  A row is halved while there are less than 8 workgroups per CU
+        // and its partitions exceed 256 tokens (below, a partition's start and the
+        // reduce cost more than they spread), or 128 for few pairs with long
+        // contexts: the last halving leaves more than half of that.  Measured on
         // gfx950 (µs per call, least partition 16 / 8 / 4 tiles of 16 tokens):
         // f32 8/8 d = 128 B = 4 L <= 200 10.1 / 11.7 / 10.9, f16 16/16 d = 256
         // B = 16 L <= 1000 50.1 / 59.0 / 58.9, f16 8/8 d = 128 B = 1 L <= 4000
@@ -813,8 +814,8 @@ void Context::decode_checked(const pam_decode_request &r, bool noalloc) {
 
 // Kernel choice, parameters and split workspace of one decode launch.  With
 // `fused` > 1 the launch serves that many consecutive layers of `layers_q` /
-// `layers_out` (same spec, shared pool): the stream-K MFMA kernel reads each K/V
-// tile once for all of their heads.
+// `layers_out` (same spec, shared pool): the MFMA kernel, stream-K or partitions, reads
+// each K/V tile once for all of their heads.
 Context::DecodePlan Context::plan_decode(const pam_decode_request &r, char *fixed, int32_t fused,
                                          const void *const *layers_q, void *const *layers_out) {
     const pam_layer_spec &l = r.layer;
@@ -864,8 +865,10 @@ Context::DecodePlan Context::plan_decode(const pam_decode_request &r, char *fixe
     return d;
 }
 
-// Layers that one stream-K launch can serve together (0: this layer cannot be
-// fused with others).
+// Layers that one MFMA launch can serve together (0: this layer cannot be fused with
+// others).  The rows are those the stream-K form takes (2048), whichever form then runs:
+// more rows fill the chip layer by layer, and the partitions of fused layers would hold
+// that many times the partials.
 int32_t Context::fusable_layers(const pam_decode_request &r) {
     const pam_layer_spec &l = r.layer;
     const int32_t G = l.num_heads / l.num_kv_heads;
@@ -1188,23 +1191,29 @@ void Context::validate_prefill(const pam_prefill_request &r) {
 }
 
 // Short prefills that the VALU kernel's workgroup form (one or two heads per
-// wave, at most 256 keys) still serves faster than the row-block kernel, whose
-// tiles cost the same for one row as for 32.  Measured on gfx950 (µs per call,
-// VALU / row blocks): f32 8/8 d = 128: 64 tokens 7.7 / 12.1, 32 after 200
-// 10.9 / 15.7, 64 after 100 15.1 / 16.3, 128 22.9 / 16.1; f32 16/8 d = 128: 64
-// 10.3 / 12.1, 64 after 100 20.5 / 16.7; f16 8/8 d = 96: 16 after 100 9.3 / 11.8,
-// 64 9.1 / 8.8; e4m3 8/4 d = 96: 8 tokens 9.9 / 8.3; f32 12/4 d = 64: 20 tokens 6.4 /
-// 7.5, 48 6.8 / 7.7, 64 10.8 / 8.1; d = 128: 8 after 100 7.8 / 13.9, 64 12.0 / 11.9, 96
-// 12.2 / 14.8; 24/4 d = 64: 16 tokens 6.8 / 7.2, 20 7.8 / 7.4; f16 12/4 d = 96: 16 7.1 / 7.8,
-// 16 after 100 9.3 / 9.9, 48 8.9 / 8.3; f32 32/8 d = 64: 4 tokens 9.8 / 6.5.
+// wave, at most 256 keys) still serves faster than the row-block kernel.  A row block's
+// time hardly moves below a few hundred keys (a tile costs the same for one row as for
+// 32: 6 to 17 us by the head size), the VALU kernel's grows with the (row, head, key)
+// triples and with the waves that an odd group needs; the lines are where the two meet in
+// triples, by the heads of a wave and the head size.  Measured on gfx950 (µs per call, VALU
+// / row blocks): f32 8/8 d = 128: 64 tokens 7.7 / 12.1, 32 after 200 10.9 / 15.7, 101 13.7 /
+// 17.1, 128 22.9 / 18; 8/4 d = 128: 95 12.0 / 16.8, 125 16.8 / 17.2; 16/8 d = 128: 64 after
+// 100 20.5 / 18; 8/8 d = 96: 95 12.7 / 13.1, 112 13.8 / 13.1; of 200 calls at 1 to 2.2 times
+// the lines the row blocks take 0.42 to 1.08 of the time.  f16 8/8 d = 96: 16 after 100 9.3 /
+// 11.8, 64 9.1 / 8.8; e4m3 8/4 d = 96: 8 tokens 9.9 / 8.3; f32 12/4 d = 64: 20 tokens 6.4 /
+// 7.5, 48 6.8 / 7.7, 64 10.8 / 8.1; 24/8 d = 128: 72 13.7 / 16.1, 75 16.2 / 17.0; 20/4 d = 128:
+// 76 12.9 / 16.8, 81 17.4 / 16.9; 24/4 d = 64: 16 tokens 6.8 / 7.2, 20 7.8 / 7.4; d = 96: 39 9.4 /
+// 9.8; d = 128: 39 9.3 / 12.7; f16 12/4 d = 96: 16 7.1 / 7.8, 16 after 100 9.3 / 9.9, 48 8.9 / 8.3;
+// f32 32/8 d = 64: 4 tokens 9.8 / 6.5.
 static bool valu_prefill_wins(const pam_layer_spec &l, int64_t rows, int64_t kv_len) {
-    const int32_t G = l.num_heads / l.num_kv_heads;
-    const int64_t pairs = rows * l.num_heads * kv_len;
+    const int32_t G = l.num_heads / l.num_kv_heads, d = l.head_dim;
+    const int64_t triples = rows * l.num_heads * kv_len;
     if (kv_len > 16 * kValuWgMaxParts || l.data_type == kFP8) return false;
-    if (l.data_type != kF32) return G % 2 == 1 && pairs < (G == 1 ? 31000 : 24000);
-    if (G <= 2) return pairs < 70000;
-    if (G % 2 == 1) return pairs < (l.head_dim > 64 ? 115000 : 48000);
-    return G % 4 == 2 && pairs < (l.head_dim > 64 ? 20000 : 9000);
+    if (l.data_type != kF32) return G % 2 == 1 && triples < (G == 1 ? 31000 : 24000);
+    auto below = [&](int64_t d64, int64_t d128, int64_t d256) { return triples < (d <= 64 ? d64 : (d <= 128 ? d128 : d256)); };
+    if (G <= 2) return below(70000, 95000, 70000);
+    if (G % 2 == 1) return below(48000, 125000, 115000);
+    return G % 4 == 2 && below(9000, 45000, 20000);
 }
 
 Context::PrefillPlan Context::plan_prefill(const pam_prefill_request &r) {

@@ -384,6 +384,25 @@ def test_f32_decode_rows_of_few_keys_stay_on_the_valu_kernel(H, hkv, d, lens, wi
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)) == valu
 
 
+@pytest.mark.parametrize("H,hkv,d,T,off,valu", [
+    (8, 4, 128, 95, 0, True), (8, 8, 128, 101, 0, True), (8, 8, 96, 112, 0, False), (8, 8, 256, 95, 0, False),
+    (8, 8, 64, 94, 0, False), (24, 8, 128, 72, 0, True), (24, 8, 128, 75, 0, False), (24, 4, 128, 39, 0, True),
+    (24, 4, 96, 9, 122, True), (24, 4, 128, 44, 0, False), (24, 4, 256, 30, 0, False),
+])
+def test_f32_prefills_of_few_keys_stay_on_the_valu_kernel(H, hkv, d, T, off, valu):
+    """By (row, head, key) triples: the same bits as with set_decode_kernel(1)."""
+    rng = np.random.default_rng(87)
+    _, k, v, bt, _ = make_case(rng, 1, H, hkv, d, 16, 0, [off + T])
+    q = rng.standard_normal((T, H, d)).astype(np.float32)
+    got = []
+    for choice in (0, 1):
+        eng = _engine()
+        eng.set_decode_kernel(choice)
+        got.append(_prefill(eng, q, to_dev(k), to_dev(v), bt[0], T, layer(H, hkv, d, 16, 0), True, off))
+    assert row_rel_err(got[0].astype(np.float64), oracle.prefill(0, q, k, v, bt[0], off, causal=True, window=0, n_threads=8)) <= TOL[0]
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)) == valu
+
+
 @pytest.mark.parametrize("dtype,H,hkv,d,B,width,most", [
     (1, 8, 1, 256, 9, 1456, 512),    # 9 to 16 pairs: 512 tokens
     (2, 16, 4, 64, 3, 1500, 512),

@@ -297,10 +297,11 @@ hipError_t launch_synth_normal(void *dst, int32_t dtype, uint64_t n, uint64_t se
 // Split-context reduce of rows whose partials are in p.part_o / p.part_ml.
 hipError_t launch_reduce(const AttnParams &p, int32_t dtype, hipStream_t stream, const KernelTable *kt);
 // Attention over blocks of query rows with f32 probabilities on the matrix units
-// (rows.hip): a prefill (kRowPrefill: 32 rows of one sequence per block) or decode
-// and ragged rows (up to 16 heads per kv-head slot), any group and block size.
-// The caller sets p.row_blocks, p.part_tokens (a multiple of 16), p.max_parts and, when max_parts > 1, the partials, which the reduce
-// launched after it merges.
+// (rows.hip): a prefill (kRowPrefill: 32 rows of one sequence per block, 16 for f32
+// above d = 128) or decode and ragged rows (up to 16 heads per kv-head slot), any group
+// and block size.  The caller sets p.row_blocks, p.part_tokens (a multiple of 16),
+// p.max_parts and, when max_parts > 1, the partials, which the reduce launched after it
+// merges.
 bool rows_supported(const AttnParams &p, int32_t dtype);
 int32_t prefill_rows_part_tokens(const AttnParams &p, int32_t dtype, int32_t cus);
 hipError_t launch_rows(const AttnParams &p, int32_t dtype, hipStream_t stream, hipEvent_t after_main,

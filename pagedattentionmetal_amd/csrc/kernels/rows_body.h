@@ -35,8 +35,8 @@
 // 784 -> 55 (44 TFLOP/s); f32 32/8 d = 128, 2048 tokens 399 (86 TFLOP/s); f16
 // 32/8 d = 96, 2048 tokens 162 (159 TFLOP/s); f16 16/16 d = 64 decode of 24 rows
 // of up to 3000 tokens 162 -> 48 (3.4 TB/s); f32 8/8 d = 128 64 rows of up to
-// 2000 128 -> 117 (4.9 TB/s); f32 32/8 one row of 5598 337 -> 12; e4m3 12/4
-// d = 128 205 rows of up to 4000 2620 -> 172.
+// 2000 130 -> 124; f32 32/8 d = 128 one row of 5598 646 -> 22; e4m3 12/4 d = 128
+// 205 rows of up to 4000 2617 -> 175.
 #pragma once
 #include "valu_body.h"
 

@@ -219,7 +219,7 @@ class Context {
     struct PrefillPlan {
         AttnParams p;
         bool dense, use_mfma;
-        bool blocks;  // row-block prefill (launch_prefill_rows)
+        bool blocks;  // row-block prefill (launch_rows)
         int64_t tmp, kv_len;
     };
     int64_t plan_prefill_rows(AttnParams &p, int32_t dtype);

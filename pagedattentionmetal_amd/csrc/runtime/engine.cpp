@@ -332,26 +332,35 @@ int32_t Context::choose_part_tokens(int64_t items_per_part, int64_t max_tiles, b
 // longest step of the call.  The host knows the rows' keys by the table's width alone.
 // Measured on gfx950 (µs per call, VALU / row blocks, tables as wide as the longest row
 // unless given): 8/8 d = 128: B = 4 L <= 200 9.5 / 10.1, B = 64 L <= 100 10.6 / 12.2, B = 128
-// L <= 200 26.0 / 30.8, B = 1 L = 360 13.3 / 13.4, B = 5 L <= 192 in a table of 384 10.4 /
-// 12.5, past 384 tokens 20% to 80% less on row blocks; d = 256 B = 4 L <= 200 14.1 / 17.0, 8
-// heads B = 4 L <= 260 in a table of 512 13.9 / 22.2, 16/16 B = 3 L <= 418 16.8 / 20.1, 4/4 B
-// = 164 L <= 288 60.4 / 74.5; 16/16 d = 64: B = 4 L <= 200 8.6 / 7.6, B = 64 15.7 / 16.7; 8/4
-// d = 128 B = 32 L <= 200 12.8 / 10.2.  Odd groups: 12/4 B = 4 L <= 200 d = 128 10.1 / 12.1,
-// d = 256 14.5 / 20.1, B = 9 L <= 240 16.8 / 22.6, B = 6 L <= 177 in a table of 352 14.5 /
-// 19.4, d = 64 9.1 / 8.3; d = 128 B = 64 L <= 100 19.4 / 8.7; 24/8 d = 128 B = 6 L <= 80 7.0 /
-// 8.4.  Ragged rows of a mixed step, where a chunk's rows share their keys in the caches,
-// one head: 367 rows of 8/8 d = 256 438 / 573, 740 of 32/32 d = 64 209 / 266, but 697 of
-// 16/16 d = 96 292 / 250 and 472 of d = 128 772 / 687.
+// L <= 200 26.0 / 30.8, B = 1 L = 360 13.3 / 13.4, B = 2 L <= 190 in a table of 384 10.2 /
+// 12.1; d = 256 B = 4 L <= 200 14.1 / 17.0, 8 heads B = 4 L <= 260 in a table of 512 13.9 /
+// 22.2, 16/16 B = 3 L <= 418 16.8 / 20.1, 4/4 B = 164 L <= 288 60.4 / 74.5; 16/16 d = 64: B = 4
+// L <= 200 8.6 / 7.6, B = 64 15.7 / 16.7; 8/4 d = 128 B = 32 L <= 200 12.8 / 10.2.  Odd
+// groups: 12/4 B = 4 L <= 200 d = 128 10.1 / 12.1, d = 256 14.5 / 20.1, B = 9 L <= 240 16.8 /
+// 22.6, d = 64 9.1 / 8.3; d = 128 B = 64 L <= 100 19.4 / 8.7; 24/8 d = 128 B = 6 L <= 80 7.0 /
+// 8.4.  350 decodes of 96 <= d <= 256, VALU over row blocks, geometric mean by (row, head)
+// pairs and tiles past 256 tokens: d > 128 G = 1 up to 64 pairs 17-32 tiles 0.87, above 64
+// 17-24 0.87, 25-32 1.02; G = 3 up to 64 pairs 17-24 0.83, above 1.26; d <= 128 up to 16 pairs
+// 17-24 0.95, 17-64 pairs 1.09, above 1.18 to 1.61.
+//
+// Ragged rows of a mixed step, one head a kv head, by the step's longest row: a chunk's
+// rows share their keys in the caches, and from 8192 pairs on a VALU row is one wave
+// without partials, which long rows wait for.  Random steps, VALU over row blocks,
+// geometric mean (range): from 16384 pairs on up to 1008 tokens 0.67 (0.40 to 0.99, 55
+// steps), past 1600 1.2 to 2.7; from 8192 up to 624 tokens 0.75 (0.53 to 0.99, 15), longer up
+// to 1.5; below that, d > 128 up to 496 tokens 0.84 (0.67 to 1.26, 52), longer 1.05 (0.65 to
+// 2.0); d <= 128 1.12 (0.78 to 3.8, 138).
 static bool valu_rows_win(const AttnParams &p, int32_t dtype, int64_t max_tiles) {
     const int64_t heads = (int64_t)p.rows * p.num_heads, d = p.head_dim;
     const int64_t G = p.num_heads / p.num_kv_heads;
     if (dtype != kF32 || G % 2 == 0) return false;
-    if (p.mode == kRowRagged && G == 1 && (d > 128 || heads >= 16384)) return true;
+    if (p.mode == kRowRagged && G == 1 && max_tiles <= (heads >= 16384 ? 64 : (heads >= 8192 ? 40 : (d > 128 ? 32 : 0))))
+        return true;
     // the line in the table's width: 256 tokens, where the VALU kernel's partitions fit one
     // workgroup; 384 for few heads; 384 to 512 at d > 128, whose tiles take longest
     int64_t most = kValuWgMaxParts;
-    if (d > 64 && heads <= (d > 128 ? 128 : 64)) most = 24;
-    if (d > 128 && G == 1) most = heads <= 128 ? 32 : 24;
+    if (d > 64 && heads <= (d > 128 ? 64 : 16)) most = 24;
+    if (d > 128 && G == 1) most = heads <= 64 ? 32 : 24;
     if (max_tiles > most) return false;
     return G == 1 ? d > 64 || heads >= 512 : d > 64 && heads <= (d > 128 ? 128 : 64);
 }

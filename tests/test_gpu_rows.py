@@ -360,10 +360,12 @@ def _wide(bt, pool, width):
     (4, 4, 256, [300] * 33, 25, False),
     (8, 8, 128, [190, 40], 24, True),         # few heads: up to 384
     (8, 8, 128, [190, 40], 25, False),
-    (8, 8, 128, [190] * 9, 24, False),
+    (8, 8, 128, [190] * 3, 24, False),
+    (4, 4, 256, [300] * 17, 32, False),
     (12, 4, 256, [177, 20], 24, True),        # an odd group
-    (12, 4, 96, [177, 20], 24, True),
-    (12, 4, 96, [177, 20] * 3, 24, False),
+    (12, 4, 256, [177, 20] * 3, 24, False),
+    (12, 4, 96, [177], 24, True),
+    (12, 4, 96, [177, 20], 24, False),
     (8, 4, 256, [177, 20], 16, False),        # an even group
 ])
 def test_f32_decode_rows_of_few_keys_stay_on_the_valu_kernel(H, hkv, d, lens, width, valu):
@@ -429,3 +431,37 @@ def test_mfma_decode_of_few_pairs_keeps_short_partitions(dtype, H, hkv, d, B, wi
     assert parts >= -(-width * 16 // most)
     ref = oracle.decode(dtype, q, k, v, bw, lens, H, k_scale=ks, v_scale=vs, n_threads=8)
     assert row_rel_err(to_host(out).astype(np.float64), ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("H,hkv,d,ctx,new,valu", [
+    (4, 4, 256, [491, 60, 0], [5, 1, 17], True),      # d > 128: up to 31 tiles of 16 tokens
+    (4, 4, 256, [492, 60, 0], [5, 1, 17], False),
+    (8, 8, 128, [300, 60, 0], [5, 1, 17], False),
+    (32, 32, 64, [40, 623], [255, 1], True),          # 8192 pairs: up to 39
+    (32, 32, 64, [40, 624], [255, 1], False),
+    (32, 32, 64, [40, 300], [254, 1], False),
+    (32, 32, 64, [40, 1007], [511, 1], True),         # 16384: up to 63
+    (32, 32, 64, [40, 1008], [511, 1], False),
+    (32, 32, 64, [40, 1007], [510, 1], False),
+    (32, 16, 64, [40, 1007], [511, 1], False),        # an even group
+])
+def test_f32_mixed_steps_of_few_keys_stay_on_the_valu_kernel(H, hkv, d, ctx, new, valu):
+    """By the longest row and the (row, head) pairs: the same bits as with set_decode_kernel(1)."""
+    import torch
+    rng = np.random.default_rng(88)
+    lens = [c + n for c, n in zip(ctx, new)]
+    _, k, v, bt, _ = make_case(rng, len(lens), H, hkv, d, 16, 0, lens)
+    q = rng.standard_normal((sum(new), H, d)).astype(np.float32)
+    got = []
+    for choice in (0, 1):
+        eng = _engine()
+        eng.set_decode_kernel(choice)
+        out = torch.full(q.shape, 7.0, dtype=torch.float32, device="cuda")
+        eng.mixed_step(to_dev(q), out, to_dev(k), to_dev(v), to_dev(bt), ctx, new, layer(H, hkv, d, 16, 0))
+        got.append(to_host(out))
+    at = 0
+    for i, n in enumerate(new):
+        ref = oracle.prefill(0, q[at:at + n], k, v, bt[i], ctx[i], causal=True, window=0, n_threads=8)
+        assert row_rel_err(got[0][at:at + n].astype(np.float64), ref) <= TOL[0]
+        at += n
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)) == valu

@@ -16,9 +16,12 @@
 // themselves before they join the row's.  Error norms against 64 bits over those of
 // the VALU rows (which add a lane's 4 products and then lanes, pairwise), geometric
 // mean and largest of 30 to 60 calls a head size: decode 0.87-0.93 and 1.05-1.16 (a few
-// outputs of one row), prefill 0.66-0.90 and 1.03.  With one chain of a tile's outputs
-// and two to eight chains of a score: 0.96-1.06 and 1.23, 0.80-1.07 and 1.40.  Time
-// against that: prefills of 2048 tokens 2-5% more, short ones 4-11%, decodes 2-5%.
+// outputs of one row), prefill 0.66-0.90 and 1.03; d > 128 0.83 and 0.98, 0.76 and 0.94.
+// With one chain of a tile's outputs and two to eight chains of a score: 0.96-1.06 and
+// 1.23, 0.80-1.07 and 1.40.  Time against that: prefills of 2048 tokens 2-5% more, short
+// ones 4-16%, decodes 2-5%, short ones up to 9%; d > 128 3-10%, 5-20% with trees of 4
+// dims there (ragged 264 rows of 16/16 d = 256 654 us, 722 and 787).  Trees of 8 dims
+// up to d = 128: decode 0.96-1.02 and 1.10, prefill 0.92-1.00 and 1.05.
 //
 // Operands come straight from the pools: a lane loads its K operand in 16-byte
 // pieces (a key's 64 bytes per instruction) and its V operand as VW consecutive
@@ -187,7 +190,9 @@ struct RowTiles {
     static constexpr int VW = F32 ? (NT % 2 == 0 ? 4 : 2) : (NT % 4 == 0 ? 8 : (NT == 2 ? 4 : 2));
     static constexpr int NU = 2 * NT / VW;
     static constexpr int LS = 32 * NT + 4;           // LDS row stride (floats)
-    static constexpr int LEAF = RB > 1 && NT > 3 ? 8 : 4;  // dot_tree's, as the registers allow
+    // dot_tree's: 8 where the registers hold no more, and where the sums are no further
+    // from 64 bits than the VALU rows' all the same (d > 128)
+    static constexpr int LEAF = NT > 4 || (RB > 1 && NT > 3) ? 8 : 4;
     typedef typename KPiece<KV>::K KOp;
     typedef typename KPiece<KV>::Q QOp;
 
